@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import concurrent.futures as cf
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -33,7 +34,7 @@ HIPFLAGS = [
 ]
 CXXFLAGS = ["-O2", "-std=c++17", "-fPIC", "-Wall", f"-I{ROOT / 'include'}"]
 
-HIP_SOURCES = ["kernel_wave.hip", "kernel_stream.hip", "kernel_tile.hip", "kernel_verify.hip", "kernel_util.hip",
+HIP_SOURCES = ["kernel_wave.hip", "kernel_wave64.hip", "kernel_stream.hip", "kernel_tile.hip", "kernel_verify.hip", "kernel_util.hip",
                "kernel_mlp.hip", "abi.cpp", "simplex_shim.cpp", "warmstart.cpp", "serve.cpp",
                "noalloc.cpp"]
 SHIM_TEST = PKG / "test_shim"  # C++ drop-in test program (tests/cpp/test_shim.cpp)
@@ -49,8 +50,34 @@ def _run(cmd: list[str]) -> None:
         print(out, file=sys.stderr)
 
 
+def _check_accumulators(asm: Path) -> None:
+    """Kernels that keep tableau entries in accumulation registers name them in inline
+    assembly only; the compiler must not place values of its own there in such a kernel."""
+    kernel, own, uses = "", False, {}
+    for line in asm.read_text().splitlines():
+        if line.startswith("_Z") and ":" in line:
+            kernel = line.split(":")[0]
+        elif "#ASMSTART" in line:
+            own = True
+        elif "#ASMEND" in line:
+            own = False
+        elif line.startswith("\t") and re.search(r"[ ,]a(\d|\[)", line.split(";")[0]):
+            uses.setdefault(kernel, {})[own] = line.strip()
+    for k, u in uses.items():
+        if len(u) == 2:
+            raise RuntimeError(f"{asm.name}: in {k} the compiler uses accumulation registers "
+                               f"({u[False]}): give the kernel more vector registers")
+
+
 def _compile(src: Path) -> Path:
     obj = OBJ / (src.name + ".o")
+    if src.name == "kernel_wave.hip":
+        _run([HIPCC, *HIPFLAGS, "--save-temps=obj", "-x", "hip", "-c", str(src), "-o", str(obj)])
+        asm = list(OBJ.glob(f"{src.stem}-hip-*{ARCH}.s"))
+        if len(asm) != 1:
+            raise RuntimeError(f"{src.name}: no device assembly to check")
+        _check_accumulators(asm[0])
+        return obj
     if src.suffix == ".hip" or src.name in ("abi.cpp", "simplex_shim.cpp", "warmstart.cpp",
                                             "serve.cpp", "noalloc.cpp"):
         cmd = [HIPCC, *HIPFLAGS, "-x", "hip", "-c", str(src), "-o", str(obj)]

@@ -82,6 +82,7 @@ struct TileTab {
   static constexpr int KB0 = 16384 / ((RCAP + CCAP) * (int)sizeof(T));
   static constexpr int KB = !BC ? 1 : KB0 < 4 ? 4 : (KB0 > 8 ? 8 : KB0);
   static constexpr bool kBlockCrash = BC;
+  static constexpr bool kEngine = false;
   static constexpr int QR = (RCAP + 63) / 64;  // rows per lane of wavefront 0
   T* cbM;    // KB x RCAP: column of target u, updated until its own step, then frozen
   T* cbP;    // KB x CCAP: row of pivot u, updated until its own step, then scaled

@@ -279,6 +279,8 @@ enum : int {
 // negative rhs below -tol; entering column: smallest max(T[0][j],0) / -T[r][j] over
 // T[r][j] < -eps_p, dual-degenerate columns by the largest |T[r][j]|) restore primal
 // feasibility; then the auxiliary phase I (if still needed) and phase II finish.
+// A backend with kEngine makes runs of pivots in one call (engine): the same pricing, ratio
+// test and pivot, in the same order, without a turn of the state machine per pivot.
 // `last`: the final pivot (row | column << 16), so that a caller can undo it: the variable
 // that left at that row is the final nonbasic variable of that column.
 template <typename T, class Tab>
@@ -389,15 +391,20 @@ __device__ __forceinline__ void run_simplex(Tab& t, int m, int n, const int8_t* 
         status = kStatusOptimal;
         break;
       }
-      T th;
-      const int r = t.ratio(s, bland, o.eps_p, th);
-      if (r < 0) {
-        if (stage == kStP2) { status = kStatusUnbounded; unb = t.nb_of(s); }
-        else status = kStatusNumeric;
-        break;
+      if constexpr (Tab::kEngine) {
+        ps = s;  // the engine makes the ratio test
+      } else {
+        T th;
+        const int r = t.ratio(s, bland, o.eps_p, th);
+        if (r < 0) {
+          if (stage == kStP2) { status = kStatusUnbounded; unb = t.nb_of(s); }
+          else status = kStatusNumeric;
+          break;
+        }
+        pr = r; ps = s;
+        deg = (th == T(0)) ? deg + 1 : 0;
       }
-      pr = r; ps = s; count_p1 = stage == kStP1;
-      deg = (th == T(0)) ? deg + 1 : 0;
+      count_p1 = stage == kStP1;
     } else {  // kStP1End
       wfin = t.get(1, 0);
       if (wfin < -o.tol) { status = kStatusInfeasible; break; }
@@ -419,7 +426,20 @@ __device__ __forceinline__ void run_simplex(Tab& t, int m, int n, const int8_t* 
         kill_after = true;
       }
     }
-    if (pr >= 0) {
+    if constexpr (Tab::kEngine) {
+      // one call makes this pivot and, in phases I and II, those that follow it
+      const bool fast = (stage == kStP1 || stage == kStP2) && !kill_after;
+      if (pr >= 0 || fast) {
+        const int it0 = it;
+        const int rc = t.engine(pr, ps, fast, stage == kStP1 ? 1 : 0, o, maxit, keep_last, it, deg, last);
+        if (count_p1) p1 += it - it0;
+        if (rc != 0) {  // no row: unbounded in phase II
+          if (stage == kStP2) { status = kStatusUnbounded; unb = t.nb_of(ps); }
+          else status = kStatusNumeric;
+          break;
+        }
+      }
+    } else if (pr >= 0) {
       t.pivot(pr, ps);
       ++it;
       if (count_p1) ++p1;

@@ -1,8 +1,8 @@
 // tuner.hpp -- per-size-bin kernel routing.
 //
 // For each LP shape the tuner picks one of:
-//   WAVE   the column-per-lane register kernel (smallest variant whose capacity covers
-//          (m+2) x (n+2) in the precision),
+//   WAVE   FP32: the matrix-core register kernel, FP64: the column-per-lane one (smallest
+//          variant whose capacity covers (m+2) x (n+2) in the precision),
 //   TILE   the 2-D register-tile kernel (smallest tile variant whose capacity covers
 //          (m+2) x (n+2) and whose registers fit),
 //   LDS    the streamed kernel with the tableau in LDS (when it fits the CU's LDS),
