@@ -34,7 +34,7 @@ HIPFLAGS = [
 ]
 CXXFLAGS = ["-O2", "-std=c++17", "-fPIC", "-Wall", f"-I{ROOT / 'include'}"]
 
-HIP_SOURCES = ["kernel_wave.hip", "kernel_wave64.hip", "kernel_stream.hip", "kernel_tile.hip", "kernel_tile64.hip",
+HIP_SOURCES = ["kernel_wave.hip", "kernel_stream.hip", "kernel_tile.hip", "kernel_tile64.hip",
                "kernel_verify.hip", "kernel_util.hip",
                "kernel_mlp.hip", "abi.cpp", "simplex_shim.cpp", "warmstart.cpp", "serve.cpp",
                "noalloc.cpp"]

@@ -679,10 +679,8 @@ static int plan_solve(blpg_ctx* ctx, blpg_batch* B, SolvePlan& P) {
       // FP64 fallback kernel of this bin
       Bin& f = fbins[i];
       f.rcap = b.rcap; f.ccap = b.ccap; f.nt = Tuner::stream_threads(b.rcap - 2, b.ccap - 2);
-      const int wv = Tuner::best_wave(b.rcap - 2, b.ccap - 2, BLPG_FP64);
       const int tv = Tuner::best_tile(b.rcap - 2, b.ccap - 2, BLPG_FP64);
-      if (wv >= 0) { f.kernel = BLPG_KERNEL_WAVE; f.variant = wv; }
-      else if (tv >= 0) { f.kernel = BLPG_KERNEL_TILE; f.variant = tv; }
+      if (tv >= 0) { f.kernel = BLPG_KERNEL_TILE; f.variant = tv; }
       else if (stream_lds_bytes(BLPG_FP64, true, f.nt, f.rcap, f.ccap) <= ctx->tuner.lds_limit() &&
                stream_max_blocks_per_cu(BLPG_FP64, true, f.nt, f.rcap, f.ccap) > 0)
         f.kernel = BLPG_KERNEL_LDS;

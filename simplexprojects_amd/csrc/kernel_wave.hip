@@ -945,6 +945,9 @@ BLPG_WAVE_VARIANTS(X)
 #undef X
 
 constexpr int kWaveVariants = 8;
+// Variant 0 is accepted in FP64 too (32 rows x 65 columns): the smallest 2-D block that holds
+// it runs it, faster than columns per lane did (27x32 x 1024: 0.109 ms against 0.113).
+constexpr int kWave64Tile = 2;
 
 int wave_variant_count() { return kWaveVariants; }
 
@@ -970,7 +973,7 @@ static const void* wave_fn(int v) {
 }
 
 int wave_max_blocks_per_cu(int precision, int v) {
-  if (precision == 0) return v == 0 ? wave64_max_blocks_per_cu() : 0;
+  if (precision == 0) return v == 0 ? tile_max_blocks_per_cu(0, kWave64Tile) : 0;
   const void* fn = wave_fn(v);
   if (!fn) return 0;
   int nb = 0;
@@ -981,7 +984,12 @@ int wave_max_blocks_per_cu(int precision, int v) {
 }
 
 hipError_t launch_wave(const TileLaunch& L, hipStream_t st) {
-  if (L.precision == 0) return L.variant == 0 ? launch_wave64(L, st) : hipErrorInvalidValue;
+  if (L.precision == 0) {
+    if (L.variant != 0) return hipErrorInvalidValue;
+    TileLaunch T = L;
+    T.variant = kWave64Tile;
+    return launch_tile(T, st);
+  }
   const void* fn = wave_fn(L.variant);
   if (!fn) return hipErrorInvalidValue;
   const int nt = wave_variant(L.precision, L.variant).nw * 64;

@@ -69,8 +69,6 @@ int wave_variant_count();
 WaveVariant wave_variant(int precision, int v);
 int wave_max_blocks_per_cu(int precision, int v);
 hipError_t launch_wave(const TileLaunch& L, hipStream_t st);
-int wave64_max_blocks_per_cu();  // the FP64 instance (kernel_wave64.hip)
-hipError_t launch_wave64(const TileLaunch& L, hipStream_t st);
 
 int tile_variant_count(int precision);
 int tile_default_variants();  // variants 0..k-1 form the static routing order
