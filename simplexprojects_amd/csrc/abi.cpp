@@ -554,7 +554,6 @@ void blpg_batch_free(blpg_ctx* ctx, blpg_batch* B) {
 struct BinPlan {
   int grid = 1;
   size_t ws_bytes = 0;
-  int64_t ws_stride = 0;
 };
 
 static int plan_bin(blpg_ctx* ctx, const Bin& b, int precision, int64_t count, BinPlan& P) {
@@ -576,11 +575,7 @@ static int plan_bin(blpg_ctx* ctx, const Bin& b, int precision, int64_t count, B
     return fail(ctx, BLPG_E_INVALID, "kernel cannot be resident (rcap %d ccap %d lds %d)",
                 b.rcap, b.ccap, (int)lds);
   P.grid = persistent_grid(ctx, per_cu, count);
-  if (!lds) {
-    const size_t esz = precision == BLPG_FP64 ? 8 : 4;
-    P.ws_stride = ((int64_t)b.rcap * b.ccap + 63) & ~63ll;
-    P.ws_bytes = (esz * (size_t)P.ws_stride * P.grid + 255) & ~(size_t)255;
-  }
+  if (!lds) P.ws_bytes = stream_ws_bytes(precision, b.rcap, b.ccap) * (size_t)P.grid;
   return BLPG_OK;
 }
 
@@ -618,7 +613,6 @@ static int launch_bin(blpg_ctx* ctx, blpg_batch* B, const Bin& b, const BinPlan&
   L.rcap = b.rcap; L.ccap = b.ccap;
   L.grid = P.grid;
   L.ws = ws;
-  L.ws_stride = P.ws_stride;
   L.warm = warm;
   HIPCHK(ctx, launch_stream(L, st));
   return BLPG_OK;

@@ -9,7 +9,7 @@
 
 namespace blpg {
 
-// Size-generic simplex kernel (kernel_stream.hip): tableau in LDS or in an HBM slab.
+// Size-generic simplex kernels (kernel_stream.hip): tableau in LDS or in an HBM slab.
 struct StreamLaunch {
   int precision;  // 0 fp64, 1 fp32
   bool lds_tab;
@@ -24,13 +24,13 @@ struct StreamLaunch {
   Out out;
   double eps_d, eps_p, tol;
   int32_t max_iter, bland_after;
-  void* ws;            // HBM slabs (lds_tab == false): grid * ws_stride elements
-  int64_t ws_stride;
+  void* ws;            // HBM slabs (lds_tab == false): grid * stream_ws_bytes
   int rcap, ccap;      // largest m+2, n+2 of the bin
   int grid;
   const int32_t* warm = nullptr;  // warm-start bases (basis pool layout), or nullptr
 };
 size_t stream_lds_bytes(int precision, bool lds_tab, int nt, int rcap, int ccap);
+size_t stream_ws_bytes(int precision, int rcap, int ccap);  // per workgroup (lds_tab == false)
 int stream_max_blocks_per_cu(int precision, bool lds_tab, int nt, int rcap, int ccap);
 hipError_t launch_stream(const StreamLaunch& L, hipStream_t st);
 

@@ -42,7 +42,9 @@ class Tuner {
     const int work = (m + 2) * (n + 2);
     if (work <= 64 * 40) return 64;
     if (work <= 128 * 48) return 128;
-    return 256;
+    // beyond LDS the kernel waits for its slab: eight wavefronts keep twice the loads in
+    // flight (64 LPs of 300x400 in FP64: 1.70 ms against 2.11)
+    return work <= 40000 ? 256 : 512;
   }
 
   // preference key: (precision, m, n) -> (kernel, variant or nt), with the measured time
