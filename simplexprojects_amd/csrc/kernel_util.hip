@@ -21,6 +21,20 @@ hipError_t launch_fill_i32(int32_t* p, int32_t v, int64_t n, hipStream_t st) {
   return hipGetLastError();
 }
 
+// two ranges to zero in one launch
+__global__ void k_clear2_i32(int32_t* p, int64_t n, int32_t* q, int64_t k) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n + k;
+       i += (int64_t)gridDim.x * blockDim.x)
+    *(i < n ? p + i : q + (i - n)) = 0;
+}
+
+hipError_t launch_clear2_i32(int32_t* p, int64_t n, int32_t* q, int64_t k, hipStream_t st) {
+  int64_t blocks = (n + k + 255) / 256;
+  if (blocks > 1024) blocks = 1024;
+  hipLaunchKernelGGL(k_clear2_i32, dim3((unsigned)blocks), dim3(256), 0, st, p, n, q, k);
+  return hipGetLastError();
+}
+
 // Expands a packed range of FP64 values: element i is vals[pref[w] + (set bits of mask[w]
 // below bit i%64)] when bit i%64 of mask[w] (w = i/64) is set, else +0.0.  pref[w] counts
 // the set bits of the words before w.
