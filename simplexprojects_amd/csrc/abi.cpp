@@ -664,6 +664,9 @@ static int plan_solve(blpg_ctx* ctx, blpg_batch* B, SolvePlan& P) {
         tv.push_back(persistent_grid(ctx, verify_max_blocks_per_cu(tier, mc, nc), cnt));
         if (tier < 2 && verify_tier_covers(tier, mc, nc, tsz)) break;
       }
+      // with a CU for every LP there is nothing to share: the last tier alone spares the
+      // launches of the others (one 105x103 LP: 9 us)
+      if (tv.size() > 2 && cnt <= ctx->props.multiProcessorCount) tv.erase(tv.begin(), tv.end() - 2);
       vstride[i] = (int64_t)verify_ws_stride(mc, nc);
       vws_off[i] = vws_total;
       if (tv[tv.size() - 2] == 2) vws_total += (size_t)vstride[i] * tv.back();

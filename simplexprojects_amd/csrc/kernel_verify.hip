@@ -39,12 +39,20 @@
 // once into LDS (row-major, odd row stride: row sweeps and column sweeps are both free of
 // bank conflicts), so the sweeps run from LDS.  Up to three tiers run in sequence on a
 // bin, each with a larger LDS budget per LP (fewer LPs per CU) and each taking the LPs the
-// previous one deferred: k_verify<128> with 31 KB, k_verify<128> with 78 KB, and
-// k_verify<256> with 150 KB, where an LP that still does not fit runs its sweeps from
-// global memory (rows batched per wavefront).
+// previous one deferred: 128 threads with 31 KB, 256 with 78 KB, and 512 with 150 KB, where
+// an LP that still does not fit runs its sweeps from global memory (rows batched per
+// wavefront).
+//
+// Few LPs: bound by the latency of some forty dependent steps (reductions, sweeps, gathers).
+// So reductions run over DPP lanes with one barrier each, and a row or column of a sweep is
+// shared by G = threads / 128 lanes.  One 105x103 LP: 32 us (42 us with 128 threads, LDS
+// swizzles and two barriers per reduction).  Many LPs: bound by the reads of A (twice, the
+// second time from the Infinity Cache) and the tableau's columns; 8192 of 105x103: 350 us
+// (360 before), about 1.1 GB from HBM.
 #include <hip/hip_runtime.h>
 
 #include <cfloat>
+#include <type_traits>
 
 #include "kernels.hpp"
 #include "simplex_device.hpp"
@@ -96,69 +104,97 @@ __host__ __device__ inline size_t stage_bytes(int m, int k, int tsz) {
   return (size_t)m * (size_t)(k | 1) * (size_t)(8 + tsz);
 }
 
+// Wavefront reductions: four DPP steps leave each row of 16 lanes with its result, the four
+// rows are read back and combined; every lane ends with the same value.  (Through
+// __shfl_xor each step is two LDS permutes: 0.9k cycles per reduction against 0.15k, and an
+// LP makes about twenty.)
+template <int CTRL>
+__device__ __forceinline__ double dpp_d(double x) {
+  const long long b = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_update_dpp((int)(b & 0xffffffffll), (int)(b & 0xffffffffll), CTRL, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp((int)(b >> 32), (int)(b >> 32), CTRL, 0xF, 0xF, false);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+__device__ __forceinline__ double lane_d(double x, int l) {
+  const long long v = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_readlane((int)(v & 0xffffffffll), l);
+  const int hi = __builtin_amdgcn_readlane((int)(v >> 32), l);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
 __device__ __forceinline__ double wmax(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off));
-  return v;
+  v = fmax(v, dpp_d<kDppXor1>(v));
+  v = fmax(v, dpp_d<kDppXor2>(v));
+  v = fmax(v, dpp_d<kDppHalfMirror>(v));
+  v = fmax(v, dpp_d<kDppMirror>(v));
+  return fmax(fmax(lane_d(v, 0), lane_d(v, 16)), fmax(lane_d(v, 32), lane_d(v, 48)));
 }
 __device__ __forceinline__ double wsum(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+  v += dpp_d<kDppXor1>(v);
+  v += dpp_d<kDppXor2>(v);
+  v += dpp_d<kDppHalfMirror>(v);
+  v += dpp_d<kDppMirror>(v);
+  return (lane_d(v, 0) + lane_d(v, 16)) + (lane_d(v, 32) + lane_d(v, 48));
+}
+// sum over groups of G neighbouring lanes (G = 1, 2, 4), in every lane of the group
+template <int G>
+__device__ __forceinline__ double gsum(double v) {
+  if constexpr (G >= 2) v += dpp_d<kDppXor1>(v);
+  if constexpr (G >= 4) v += dpp_d<kDppXor2>(v);
   return v;
 }
 
-// workgroup reductions through `red` (NT/64 doubles), uniform result
+// Workgroup reductions, uniform result.  Two buffers in turn, so each takes one barrier.
 template <int NT>
-__device__ __forceinline__ double bmax(double v, double* red) {
+struct Red {
+  static constexpr int NW = NT / 64;
+  double* buf;  // 4 * NW doubles
+  int ph;
+  __device__ __forceinline__ double* next() {
+    ph ^= 1;
+    return buf + ph * 2 * NW;
+  }
+};
+template <int NT>
+__device__ __forceinline__ double bmax(double v, Red<NT>& red) {
+  double* b = red.next();
   v = wmax(v);
+  if ((threadIdx.x & 63) == 0) b[threadIdx.x >> 6] = v;
   __syncthreads();
-  if constexpr (NT == 64) {
-    return v;
-  } else {
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    double r = red[0];
+  double r = b[0];
 #pragma unroll
-    for (int w = 1; w < NT / 64; ++w) r = fmax(r, red[w]);
-    return r;
-  }
+  for (int w = 1; w < NT / 64; ++w) r = fmax(r, b[w]);
+  return r;
 }
-// two maxima in one reduction (red: 2 * NT/64 doubles)
+// two maxima in one reduction
 template <int NT>
-__device__ __forceinline__ void bmax2(double& a, double& b, double* red) {
+__device__ __forceinline__ void bmax2(double& a, double& c, Red<NT>& red) {
+  double* b = red.next();
   a = wmax(a);
-  b = wmax(b);
-  __syncthreads();
-  if constexpr (NT != 64) {
-    if ((threadIdx.x & 63) == 0) {
-      red[threadIdx.x >> 6] = a;
-      red[NT / 64 + (threadIdx.x >> 6)] = b;
-    }
-    __syncthreads();
-    double ra = red[0], rb = red[NT / 64];
-#pragma unroll
-    for (int w = 1; w < NT / 64; ++w) {
-      ra = fmax(ra, red[w]);
-      rb = fmax(rb, red[NT / 64 + w]);
-    }
-    a = ra;
-    b = rb;
+  c = wmax(c);
+  if ((threadIdx.x & 63) == 0) {
+    b[threadIdx.x >> 6] = a;
+    b[NT / 64 + (threadIdx.x >> 6)] = c;
   }
+  __syncthreads();
+  double ra = b[0], rc = b[NT / 64];
+#pragma unroll
+  for (int w = 1; w < NT / 64; ++w) {
+    ra = fmax(ra, b[w]);
+    rc = fmax(rc, b[NT / 64 + w]);
+  }
+  a = ra;
+  c = rc;
 }
 template <int NT>
-__device__ __forceinline__ double bsum(double v, double* red) {
+__device__ __forceinline__ double bsum(double v, Red<NT>& red) {
+  double* b = red.next();
   v = wsum(v);
+  if ((threadIdx.x & 63) == 0) b[threadIdx.x >> 6] = v;
   __syncthreads();
-  if constexpr (NT == 64) {
-    return v;
-  } else {
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    double r = red[0];
+  double r = b[0];
 #pragma unroll
-    for (int w = 1; w < NT / 64; ++w) r += red[w];
-    return r;
-  }
+  for (int w = 1; w < NT / 64; ++w) r += b[w];
+  return r;
 }
 
 // compacts {i < cnt : pred(i)} in ascending order into out (and key(i) into out2);
@@ -173,14 +209,13 @@ __device__ int compact(int cnt, Pred pred, Key key, int* out, int* out2, int* re
     const unsigned long long bal = __ballot(p);
     const int before = __popcll(bal & ((1ull << lane) - 1ull));
     int off = base, tot = 0;
-    if constexpr (NT == 64) {
-      tot = __popcll(bal);
-    } else {
-      __syncthreads();
-      if (lane == 0) red_i[w] = __popcll(bal);
-      __syncthreads();
-      for (int q = 0; q < w; ++q) off += red_i[q];
-      for (int q = 0; q < NT / 64; ++q) tot += red_i[q];
+    __syncthreads();
+    if (lane == 0) red_i[w] = __popcll(bal);
+    __syncthreads();
+    for (int q = 0; q < NT / 64; ++q) {
+      const int c = red_i[q];
+      off += q < w ? c : 0;
+      tot += c;
     }
     if (p) {
       out[off + before] = i;
@@ -196,12 +231,15 @@ __device__ int compact(int cnt, Pred pred, Key key, int* out, int* out2, int* re
 
 // Checks one LP with NT threads.  wsp: the per-LP vectors; stg: `stage_cap` bytes of LDS
 // for the staged blocks.  Returns false (and writes nothing) when the blocks do not fit
-// and `defer` is set or NT < 256: the caller hands the LP to the four-wavefront kernel.
-template <typename TT, int NT>
+// and `defer` is set or this is not the last tier: the caller hands the LP on.
+// LAST: the last tier, which defers nothing.  Rows of a sweep take G = NT / 128 neighbouring
+// lanes each.
+template <typename TT, int NT, bool LAST>
 __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ pool,
                           const int8_t* __restrict__ spool, Out out, Check chk, double tol,
                           int fp32_source, char* wsp, char* stg, int64_t stage_cap, bool defer,
-                          double* red, int* red_i, int32_t* fail_list, int32_t* fail_count) {
+                          Red<NT>& red, int* red_i, int32_t* fail_list, int32_t* fail_count) {
+  constexpr int G = NT / 128;
   const int tid = threadIdx.x;
   const int m = D.m, n = D.n, R = m + 2, C = n + 2;
   const double* A = pool + D.a;
@@ -248,7 +286,7 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
       kl += (v >= 0 && v < n) ? 1 : 0;
       xl |= v == n + m ? 1 : 0;
     }
-    if (defer || NT < 256) {
+    if (defer || !LAST) {
       // an LP this tier hands on is decided from its basis alone (the size of its staged
       // blocks), before the rest of the bookkeeping
       const int ke = (int)bsum<NT>((double)kl, red) + ((infeas && bmax<NT>((double)xl, red) > 0) ? 1 : 0);
@@ -280,9 +318,9 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
   }
   const int kk = kq > k ? kq : k;  // columns of the staged blocks
   const bool fits = checkable && !bad && stage_bytes(m, kk, (int)sizeof(TT)) <= (size_t)stage_cap;
-  if (checkable && !bad && !fits && (defer || NT < 256)) return false;
-  // the first-pass kernel only ever runs staged (its global-memory sweeps are not built)
-  const bool staged = NT < 256 || fits;
+  if (checkable && !bad && !fits && (defer || !LAST)) return false;
+  // only the last tier's kernel has the global-memory sweeps
+  const bool staged = !LAST || fits;
 
   double bm = 0, cm = 0;
   for (int i = tid; i < m; i += NT) bm = fmax(bm, fabs(b[i]));
@@ -312,56 +350,33 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
     for (int a = tid; a < k; a += NT) cS[a] = c[S[a]];
     if (staged && kk > 0) {
       // one pass of gathers; thread (tp, ta) copies rows tp, tp + per, ... of column ta,
-      // eight rows per step with all loads of a step in flight together.  128 threads: the
-      // last step's rows past m re-read row m - 1 and are not stored; 256 threads (whose
-      // registers the clamped step would spill): the rows left after the full steps one
-      // at a time.  (With x0 basic the T block has one column more than the A block; its
-      // A column a = k is a copy of column k-1, or of column 0 of A, never read.)
+      // eight rows per step with all loads of a step in flight together; the last step's rows
+      // past m re-read row m - 1 and are not stored.  (With x0 basic the T block has one
+      // column more than the A block; its A column a = k is a copy of column k-1, or of
+      // column 0 of A, never read.)
       const int per = kk >= NT ? 1 : NT / kk;
       const int ta = kk >= NT ? tid : tid % kk, tp = kk >= NT ? 0 : tid / kk;
       if (tp < per) {
         for (int a = ta; a < kk; a += NT) {
           const int ca = a < k ? S[a] : (k > 0 ? S[k - 1] : 0), cp = Pcol[a];
-          if constexpr (NT < 256) {
-            for (int p = tp; p < m; p += 8 * per) {
-              double av[8];
-              TT tv[8];
-              int8_t sv[8];
+          for (int p = tp; p < m; p += 8 * per) {
+            double av[8];
+            TT tv[8];
+            int8_t sv[8];
 #pragma unroll
-              for (int u = 0; u < 8; ++u) {
-                const int pu = min(p + u * per, m - 1);
-                av[u] = A[(int64_t)pu * n + ca];
-                tv[u] = T[(int64_t)(2 + pu) * C + cp];
-                sv[u] = sense ? sense[pu] : (int8_t)0;
-              }
-#pragma unroll
-              for (int u = 0; u < 8; ++u) {
-                const int pu = p + u * per;
-                if (pu < m) {
-                  AB[pu * kpad + a] = (sv[u] == 2 ? -1.0 : 1.0) * av[u];
-                  TB[pu * kpad + a] = tv[u];
-                }
-              }
+            for (int u = 0; u < 8; ++u) {
+              const int pu = min(p + u * per, m - 1);
+              av[u] = A[(int64_t)pu * n + ca];
+              tv[u] = T[(int64_t)(2 + pu) * C + cp];
+              sv[u] = sense ? sense[pu] : (int8_t)0;
             }
-          } else {
-            int p = tp;
-            for (; p + 7 * per < m; p += 8 * per) {
-              double av[8];
-              TT tv[8];
 #pragma unroll
-              for (int u = 0; u < 8; ++u) {
-                av[u] = A[(int64_t)(p + u * per) * n + ca];
-                tv[u] = T[(int64_t)(2 + p + u * per) * C + cp];
+            for (int u = 0; u < 8; ++u) {
+              const int pu = p + u * per;
+              if (pu < m) {
+                AB[pu * kpad + a] = (sv[u] == 2 ? -1.0 : 1.0) * av[u];
+                TB[pu * kpad + a] = tv[u];
               }
-#pragma unroll
-              for (int u = 0; u < 8; ++u) {
-                AB[(p + u * per) * kpad + a] = sg(p + u * per) * av[u];
-                TB[(p + u * per) * kpad + a] = tv[u];
-              }
-            }
-            for (; p < m; p += per) {
-              AB[p * kpad + a] = sg(p) * A[(int64_t)p * n + ca];
-              TB[p * kpad + a] = T[(int64_t)(2 + p) * C + cp];
             }
           }
         }
@@ -370,30 +385,50 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
     __syncthreads();
     const int lane = tid & 63, wave = tid >> 6;
 
+    // Every sum is formed in an order that does not depend on the tier: four classes (index
+    // mod 4), each summed in ascending order, then (0 + 1) + (2 + 3).  A lane or thread takes
+    // 4 / G neighbouring classes.  (Column sums: eight classes.)
+    constexpr int NC = 4 / G;
+    // sum_a M[a] w[a] over a < k by the G lanes of a row
+    auto row_dot = [&](const auto* M) {
+      const int g = tid % G * NC;
+      double s[NC];
+#pragma unroll
+      for (int i = 0; i < NC; ++i) s[i] = 0;
+      int a = g;
+      for (; a + 8 <= k; a += 8) {
+#pragma unroll
+        for (int i = 0; i < NC; ++i) s[i] = fma((double)M[a + i], w[a + i], s[i]);
+#pragma unroll
+        for (int i = 0; i < NC; ++i) s[i] = fma((double)M[a + 4 + i], w[a + 4 + i], s[i]);
+      }
+      for (; a < k; a += 4) {
+#pragma unroll
+        for (int i = 0; i < NC; ++i)
+          if (a + i < k) s[i] = fma((double)M[a + i], w[a + i], s[i]);
+      }
+      if constexpr (NC == 4) return (s[0] + s[1]) + (s[2] + s[3]);
+      else if constexpr (NC == 2) return gsum<G>(s[0] + s[1]);
+      else return gsum<G>(s[0]);
+    };
     // r = rhs - B v for the basis matrix B of [A' I]; rhs is b' (ray == false) or the
     // entering column a'_e.  Returns the thread's max |r| (reduced by the caller).
     auto resid = [&](const double* vb, bool ray, int e) {
       double rl = 0;
       if (staged) {
-        // one thread per constraint row over the staged block
+        // G lanes per constraint row over the staged block
         for (int a = tid; a < k; a += NT) w[a] = vb[Srow[a]];
         __syncthreads();
-        for (int p = tid; p < m; p += NT) {
-          const double* ABp = AB + p * kpad;
-          double s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-          int a = 0;
-          for (; a + 4 <= k; a += 4) {
-            s0 = fma(ABp[a], w[a], s0);
-            s1 = fma(ABp[a + 1], w[a + 1], s1);
-            s2 = fma(ABp[a + 2], w[a + 2], s2);
-            s3 = fma(ABp[a + 3], w[a + 3], s3);
+        for (int p0 = 0; p0 < m; p0 += NT / G) {
+          const int p = p0 + tid / G, pc = p < m ? p : m - 1;
+          const double tot = row_dot(AB + pc * kpad);
+          if (p < m && tid % G == 0) {
+            const int q = rowof[n + p];
+            const double rhs = ray ? ae[p] : bp[p];
+            const double val = rhs - tot - (q >= 0 ? vb[q] : 0.0);
+            r[p] = val;
+            rl = fmax(rl, fabs(val));
           }
-          for (; a < k; ++a) s0 = fma(ABp[a], w[a], s0);
-          const int q = rowof[n + p];
-          const double rhs = ray ? ae[p] : bp[p];
-          const double val = rhs - ((s0 + s1) + (s2 + s3)) - (q >= 0 ? vb[q] : 0.0);
-          r[p] = val;
-          rl = fmax(rl, fabs(val));
         }
       } else {
         // from global memory: each wavefront takes kRB rows at a time (kRB independent
@@ -434,19 +469,13 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
       if (staged) {
         for (int a = tid; a < k; a += NT) w[a] = r[Pn[a]];
         __syncthreads();
-        for (int i = tid; i < m; i += NT) {
-          const TT* TBi = TB + i * kpad;
-          double s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-          int a = 0;
-          for (; a + 4 <= k; a += 4) {
-            s0 = fma((double)TBi[a], w[a], s0);
-            s1 = fma((double)TBi[a + 1], w[a + 1], s1);
-            s2 = fma((double)TBi[a + 2], w[a + 2], s2);
-            s3 = fma((double)TBi[a + 3], w[a + 3], s3);
+        for (int i0 = 0; i0 < m; i0 += NT / G) {
+          const int i = i0 + tid / G, ic = i < m ? i : m - 1;
+          const double tot = row_dot(TB + ic * kpad);
+          if (i < m && tid % G == 0) {
+            const int v = bs[i];
+            vb[i] += tot + (v >= n ? r[v - n] : 0.0);
           }
-          for (; a < k; ++a) s0 = fma((double)TBi[a], w[a], s0);
-          const int v = bs[i];
-          vb[i] += ((s0 + s1) + (s2 + s3)) + (v >= n ? r[v - n] : 0.0);
         }
       } else {
         for (int i0 = wave * kRB; i0 < m; i0 += (NT / 64) * kRB) {
@@ -475,33 +504,99 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
       }
       __syncthreads();
     };
-    // column sums over a staged block: emit(a, sum_p M[p][a] v[p]) for a < cnt.  Thread
-    // (tp, ta) sums rows tp, tp + per, ... of column ta (all NT threads busy when cnt < NT);
-    // the per partials of a column are then added in order.
+    // column sums over a staged block: emit(a, sum_p M[p][a] v[p]) for a < cnt.  Eight classes
+    // of rows (index mod 8) in one, two, four or eight threads per column (as many as there
+    // are); their sums meet in LDS.
     auto colsum = [&](const auto* M, const double* v, int cnt, auto&& emit) {
-      const int pc = part_cap(m, NT) / kpad;
-      const int per = cnt >= NT || cnt == 0 ? 1 : (NT / cnt < pc ? NT / cnt : pc);
-      const int ta = cnt >= NT || cnt == 0 ? tid : tid % cnt,
-                tp = cnt >= NT || cnt == 0 ? 0 : tid / cnt;
-      if (cnt > 0 && tp < per) {
-        for (int a = ta; a < cnt; a += NT) {
-          double s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-          int p = tp;
-          for (; p + 3 * per < m; p += 4 * per) {
-            s0 = fma((double)M[p * kpad + a], v[p], s0);
-            s1 = fma((double)M[(p + per) * kpad + a], v[p + per], s1);
-            s2 = fma((double)M[(p + 2 * per) * kpad + a], v[p + 2 * per], s2);
-            s3 = fma((double)M[(p + 3 * per) * kpad + a], v[p + 3 * per], s3);
-          }
-          for (; p < m; p += per) s0 = fma((double)M[p * kpad + a], v[p], s0);
-          part[tp * kpad + a] = (s0 + s1) + (s2 + s3);
+      // the sum over the classes c0 .. c0 + NCL - 1 of column Ma
+      auto share = [&](auto ncl, const auto* Ma, int c0) {
+        constexpr int NCL = decltype(ncl)::value;
+        double t[NCL];
+#pragma unroll
+        for (int i = 0; i < NCL; ++i) t[i] = 0;
+        int p = c0;
+        for (; p + NCL <= m; p += 8)
+#pragma unroll
+          for (int i = 0; i < NCL; ++i) t[i] = fma((double)Ma[(p + i) * kpad], v[p + i], t[i]);
+        if constexpr (NCL > 1) {
+#pragma unroll
+          for (int i = 0; i < NCL; ++i)
+            if (p + i < m) t[i] = fma((double)Ma[(p + i) * kpad], v[p + i], t[i]);
         }
+        if constexpr (NCL == 8) return ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
+        else if constexpr (NCL == 4) return (t[0] + t[1]) + (t[2] + t[3]);
+        else if constexpr (NCL == 2) return t[0] + t[1];
+        else return t[0];
+      };
+      using std::integral_constant;
+      if (2 * cnt > NT) {
+        for (int a = tid; a < cnt; a += NT) emit(a, share(integral_constant<int, 8>{}, M + a, 0));
+        return;
       }
+      const int sh = cnt == 0 ? 0 : 4 * cnt > NT ? 1 : 8 * cnt > NT ? 2 : 3;  // log2(threads)
+      const int ta = cnt == 0 ? 0 : tid % cnt, tp = cnt == 0 ? 1 : tid / cnt;
+      if (tp < (1 << sh))
+        part[tp * cnt + ta] = sh == 3   ? share(integral_constant<int, 1>{}, M + ta, tp)
+                              : sh == 2 ? share(integral_constant<int, 2>{}, M + ta, 2 * tp)
+                                        : share(integral_constant<int, 4>{}, M + ta, 4 * tp);
       __syncthreads();
-      for (int a = tid; a < cnt; a += NT) {
-        double sum = 0;
-        for (int q = 0; q < per; ++q) sum += part[q * kpad + a];
-        emit(a, sum);
+      if (tid < cnt) {
+        double q[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) q[i] = i < (1 << sh) ? part[i * cnt + tid] : 0.0;
+        emit(tid, sh == 3   ? ((q[0] + q[1]) + (q[2] + q[3])) + ((q[4] + q[5]) + (q[6] + q[7]))
+                  : sh == 2 ? (q[0] + q[1]) + (q[2] + q[3])
+                            : q[0] + q[1]);
+      }
+    };
+    // f(j, sum over rows of A[p][j] w[p]) for every structural column j: G threads per column,
+    // 16 loads in flight each; their sums meet in LDS
+    auto a_columns = [&](auto&& f) {
+      const int u = tid / 128, jj = tid % 128;
+      constexpr int ST = 16 / NC;  // steps of four rows per batch of loads
+      for (int j0 = 0; j0 < n; j0 += 128) {
+        const int j = j0 + jj;
+        double t[NC];
+#pragma unroll
+        for (int i = 0; i < NC; ++i) t[i] = 0;
+        if (j < n) {
+          int p0 = u * NC;
+          for (; p0 + 4 * (ST - 1) + NC <= m; p0 += 4 * ST) {
+            double av[ST][NC];
+#pragma unroll
+            for (int q = 0; q < ST; ++q)
+#pragma unroll
+              for (int i = 0; i < NC; ++i) av[q][i] = A[(int64_t)(p0 + 4 * q + i) * n + j];
+#pragma unroll
+            for (int q = 0; q < ST; ++q)
+#pragma unroll
+              for (int i = 0; i < NC; ++i) t[i] = fma(av[q][i], w[p0 + 4 * q + i], t[i]);
+          }
+          // the rows left: those past m re-read row m - 1 and are not used
+          if (p0 < m) {
+            double av[ST][NC];
+#pragma unroll
+            for (int q = 0; q < ST; ++q)
+#pragma unroll
+              for (int i = 0; i < NC; ++i) av[q][i] = A[(int64_t)min(p0 + 4 * q + i, m - 1) * n + j];
+#pragma unroll
+            for (int q = 0; q < ST; ++q)
+#pragma unroll
+              for (int i = 0; i < NC; ++i)
+                if (p0 + 4 * q + i < m) t[i] = fma(av[q][i], w[p0 + 4 * q + i], t[i]);
+          }
+        }
+        double tot;
+        if constexpr (NC == 4) {
+          tot = (t[0] + t[1]) + (t[2] + t[3]);
+        } else {
+          __syncthreads();
+          part[tid] = NC == 2 ? t[0] + t[NC - 1] : t[0];
+          __syncthreads();
+          tot = G == 2 ? part[jj] + part[128 + jj]
+                       : (part[jj] + part[128 + jj]) + (part[(256 + jj) % NT] + part[(384 + jj) % NT]);
+        }
+        if (u == 0 && j < n) f(j, tot);
       }
     };
     // refinement: stops at the rounding floor, after kMaxSweeps, or when a sweep no
@@ -602,27 +697,10 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
       }
       __syncthreads();
       double vg = 0;
-      for (int j = tid; j < n; j += NT) {
-        // one column per thread, 16 independent row loads in flight per step
-        double s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-        int p = 0;
-        for (; p + 16 <= m; p += 16) {
-          double av[16];
-  #pragma unroll
-          for (int u = 0; u < 16; ++u) av[u] = A[(int64_t)(p + u) * n + j];
-  #pragma unroll
-          for (int u = 0; u < 16; u += 4) {
-            s0 = fma(av[u], w[p + u], s0);
-            s1 = fma(av[u + 1], w[p + u + 1], s1);
-            s2 = fma(av[u + 2], w[p + u + 2], s2);
-            s3 = fma(av[u + 3], w[p + u + 3], s3);
-          }
-        }
-        for (; p < m; ++p) s0 = fma(A[(int64_t)p * n + j], w[p], s0);
-        vg = fmax(vg, -((s0 + s1) + (s2 + s3)));
-      }
+      a_columns([&](int, double tot) { vg = fmax(vg, -tot); });
       double hp = 0;
-      for (int p = tid; p < m; p += NT) hp = fma(b[p], w[p], hp);
+      if (tid < 128)
+        for (int p = tid; p < m; p += 128) hp = fma(b[p], w[p], hp);
       bmax2<NT>(vg, yneg, red);
       const double h = bsum<NT>(hp, red);
       const double gs = am * ym;
@@ -723,25 +801,9 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
         for (int p = tid; p < m; p += NT) w[p] = sg(p) * y[p];
         __syncthreads();
         double dvv = 0;
-        for (int j = tid; j < n; j += NT) {
-          // one column per thread, 16 independent row loads in flight per step
-          double s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-          int p = 0;
-          for (; p + 16 <= m; p += 16) {
-            double av[16];
-    #pragma unroll
-            for (int u = 0; u < 16; ++u) av[u] = A[(int64_t)(p + u) * n + j];
-    #pragma unroll
-            for (int u = 0; u < 16; u += 4) {
-              s0 = fma(av[u], w[p + u], s0);
-              s1 = fma(av[u + 1], w[p + u + 1], s1);
-              s2 = fma(av[u + 2], w[p + u + 2], s2);
-              s3 = fma(av[u + 3], w[p + u + 3], s3);
-            }
-          }
-          for (; p < m; ++p) s0 = fma(A[(int64_t)p * n + j], w[p], s0);
-          if (rowof[j] < 0) dvv = fmax(dvv, c[j] - ((s0 + s1) + (s2 + s3)));
-        }
+        a_columns([&](int j, double tot) {
+          if (rowof[j] < 0) dvv = fmax(dvv, c[j] - tot);
+        });
         for (int p = tid; p < m; p += NT)
           if (colp[p] >= 0 && !is_eq(p)) dvv = fmax(dvv, -y[p]);
         rd = fmax(bmax<NT>(dvv, red), rres_d) / (1.0 + cm + am * ym);
@@ -750,7 +812,8 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
 
       // objective of the FP64 basic solution
       double zp = 0;
-      for (int a = tid; a < k; a += NT) zp = fma(c[S[a]], x[Srow[a]], zp);
+      if (tid < 128)
+        for (int a = tid; a < k; a += 128) zp = fma(c[S[a]], x[Srow[a]], zp);
       const double zsum = bsum<NT>(zp, red);
       kx = k;
       if (status == kStatusOptimal) {
@@ -786,7 +849,8 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
           }
           viol = bmax<NT>(viol, red);
           double part = 0;
-          for (int a = tid; a < k; a += NT) part = fma(c[S[a]], dv[Srow[a]], part);
+          if (tid < 128)
+            for (int a = tid; a < k; a += 128) part = fma(c[S[a]], dv[Srow[a]], part);
           const double gain = (e < n ? c[e] : 0.0) - bsum<NT>(part, red);
           good = viol <= tol * (1.0 + dmax) && rres2 <= tol * (1.0 + am * dmax) &&
                  gain > tol * (1.0 + cm * (1.0 + dmax));
@@ -841,10 +905,12 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
 // workgroup that draws slow LPs takes fewer, so the launch ends with the LPs, not with the
 // unluckiest fixed share.  Dynamic LDS: [vectors (if lds_scratch)][stage_cap bytes].  With
 // a defer_list, LPs whose staged blocks exceed stage_cap go to it (the next tier takes
-// them); NT < 256 always defers them.
-// NT = 128: at most 168 VGPRs, three waves per SIMD (five LPs per CU, as its LDS allows)
-template <int NT>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 128 ? 3 : 1))) void k_verify(const LpDesc* __restrict__ desc,
+// them); only the last tier has nothing to defer to.
+// Tier 0: at most 168 VGPRs, three waves per SIMD (five LPs per CU, as its LDS allows); the
+// others two (two LPs of four wavefronts, one of eight; held to 168 the second tier spills
+// 60 registers).
+template <typename TT, int NT, bool LAST>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 128 ? 3 : 2))) void k_verify(const LpDesc* __restrict__ desc,
                                                const double* __restrict__ pool,
                                                const int8_t* __restrict__ spool,
                                                const int32_t* __restrict__ idx, int32_t count,
@@ -857,7 +923,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 128 ? 
                                                int32_t* defer_count) {
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ int s_q;
-  __shared__ double red[2 * (NT / 64)];
+  __shared__ double red_buf[4 * (NT / 64)];
+  Red<NT> red;
+  red.buf = red_buf;
+  red.ph = 0;
   __shared__ int red_i[NT / 64];
   char* wsp = lds_scratch ? (char*)smem : ws + (int64_t)blockIdx.x * ws_stride;
   char* stg = (char*)smem + (lds_scratch ? vec_bytes : 0);
@@ -871,13 +940,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 128 ? 
     if (q >= count) break;
     const int lp = idx ? idx[q] : q;
     const LpDesc D = desc[lp];
-    // the dump's precision: FP32 tableau, or FP64 for FP64 solves and FP64 fallbacks
-    const bool done =
-        fp32_source
-            ? verify_lp<float, NT>(lp, D, pool, spool, out, chk, tol, 1, wsp, stg, stage_cap,
-                                   defer, red, red_i, fail_list, fail_count)
-            : verify_lp<double, NT>(lp, D, pool, spool, out, chk, tol, 0, wsp, stg, stage_cap,
-                                    defer, red, red_i, fail_list, fail_count);
+    const bool done = verify_lp<TT, NT, LAST>(lp, D, pool, spool, out, chk, tol, fp32_source, wsp, stg,
+                                              stage_cap, defer, red, red_i, fail_list, fail_count);
     if (!done && threadIdx.x == 0 && defer_list) defer_list[atomicAdd(defer_count, 1)] = lp;
   }
 }
@@ -886,11 +950,11 @@ namespace {
 // Tiers of the check, run in sequence on a bin; each takes the LPs the previous one
 // deferred.  0: 128 threads and 31 KB per LP (5 LPs per CU: at 32 KB the fifth one is not
 // resident although the occupancy query counts it), for LPs with few basic
-// structurals; 1: 128 threads, 78 KB (2 per CU; 256 threads would need 256 VGPRs and leave
-// one); 2: 256 threads, 150 KB (1 per CU), which
+// structurals; 1: 256 threads, 78 KB (2 per CU); 2: 512 threads, 150 KB (1 per CU), which
 // defers nothing (global-memory sweeps for what does not fit, vectors in HBM when even
-// they exceed 48 KB).
-constexpr int kTierNT[3] = {128, 128, 256};
+// they exceed 48 KB).  LDS sets how many LPs a CU checks at once, so the larger tiers give
+// each LP more threads: eight wavefronts per CU in both.
+constexpr int kTierNT[3] = {128, 256, 512};
 constexpr size_t kTierLds[3] = {31 * 1024, 78 * 1024, 150 * 1024};
 constexpr size_t kVecLdsMax = 48 * 1024;
 
@@ -909,9 +973,12 @@ void lds_plan(int tier, int mcap, int ncap, int64_t& stage_cap, size_t& lds) {
   if (stage_cap > most) stage_cap = most;
   lds = vb + (size_t)stage_cap;
 }
+// TT: the dump's precision (FP32 tableaux, or FP64 of FP64 solves and fallbacks)
+template <typename TT>
 const void* kernel_of(int tier) {
-  return kTierNT[tier] == 128 ? reinterpret_cast<const void*>(&k_verify<128>)
-                              : reinterpret_cast<const void*>(&k_verify<256>);
+  return tier == 0 ? reinterpret_cast<const void*>(&k_verify<TT, 128, false>)
+         : tier == 1 ? reinterpret_cast<const void*>(&k_verify<TT, 256, false>)
+                     : reinterpret_cast<const void*>(&k_verify<TT, 512, true>);
 }
 }  // namespace
 
@@ -940,7 +1007,7 @@ int verify_max_blocks_per_cu(int tier, int mcap, int ncap) {
   int64_t sc;
   size_t lds;
   lds_plan(tier, mcap, ncap, sc, lds);
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel_of(tier), kTierNT[tier], lds) !=
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel_of<double>(tier), kTierNT[tier], lds) !=
       hipSuccess)
     return 0;
   return nb;
@@ -948,7 +1015,8 @@ int verify_max_blocks_per_cu(int tier, int mcap, int ncap) {
 
 // HBM vectors per workgroup of the last tier when they exceed the LDS share (0: LDS)
 size_t verify_ws_stride(int mcap, int ncap) {
-  return vec_in_lds(mcap, ncap, 256) ? 0 : (vec_bytes(mcap, ncap, 256) + 255) & ~(size_t)255;
+  const int nt = kTierNT[2];
+  return vec_in_lds(mcap, ncap, nt) ? 0 : (vec_bytes(mcap, ncap, nt) + 255) & ~(size_t)255;
 }
 
 hipError_t launch_verify(const VerifyLaunch& V, hipStream_t st) {
@@ -974,7 +1042,7 @@ hipError_t launch_verify(const VerifyLaunch& V, hipStream_t st) {
                   (void*)&V.tol, (void*)&V.fp32_source, (void*)&ws, (void*)&stride,
                   (void*)&lds_scratch, (void*)&vb, (void*)&stage_cap, (void*)&V.queue,
                   (void*)&V.fail_list, (void*)&V.fail_count, (void*)&dl, (void*)&dc};
-  return hipLaunchKernel(kernel_of(V.tier), dim3(V.grid), dim3(nt), args, lds, st);
+  return hipLaunchKernel(V.fp32_source ? kernel_of<float>(V.tier) : kernel_of<double>(V.tier), dim3(V.grid), dim3(nt), args, lds, st);
 }
 
 }  // namespace blpg
