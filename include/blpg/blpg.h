@@ -165,8 +165,9 @@ void blpg_batch_free(blpg_ctx *ctx, blpg_batch *batch);
 int blpg_batch_repack(blpg_ctx *ctx, blpg_batch *batch, const blpg_lp *lps, int64_t count);
 
 /* Bulk results of the last blpg_batch_solve without per-LP copies: waits for the solve,
- * copies the batch's results with one DMA into host memory the batch owns (pinned) and
- * points `res` at it.  The arrays stay valid until the next solve, fetch or free of the
+ * points `res` at host memory the batch owns (pinned), which the first fetch of a batch
+ * fills with one DMA and the check of later solves as they run (without a check: the DMA).
+ * The arrays stay valid until the next solve, fetch or free of the
  * batch.  LP k's x is x[x_offset[k] .. + n_k), its basis basis[basis_offset[k] .. + m_k). */
 typedef struct {
   int64_t count;

@@ -704,6 +704,13 @@ static int plan_workspaces(blpg_ctx* ctx, blpg_batch* B) {
 static constexpr int kEvEnd = 65;
 static constexpr int kEvWsStart = 66, kEvWsEnd = 67;  // learned warm start inference
 
+// Whether solves of the batch write its host copy of the results (see Check).  The per-LP
+// numbers too (eleven small writes an LP): leaving those to a copy measured the same at
+// 4096 and 8192 LPs, and cost a single LP the copy's 15 us.
+static bool mirrors(const blpg_ctx* ctx, const blpg_batch* B) {
+  return B->h_res && !B->d_count && (ctx->opt.verify || ctx->opt.precision == BLPG_FP32);
+}
+
 // Enqueues one solve of the batch on the context stream (and the aux streams it forks
 // to).  With `timing` every stage is bracketed by timing events; without, only the
 // fork / join events are recorded, so the sequence can be captured into a hipGraph.
@@ -730,6 +737,18 @@ static int enqueue_solve(blpg_ctx* ctx, blpg_batch* B, bool timing, bool copy) {
   std::vector<size_t>& ws_off = P.ws_off;
   std::vector<size_t>& fws_off = P.fws_off;
   std::vector<size_t>& vws_off = P.vws_off;
+
+  // with a host copy at hand (a fetch allocated it) the check writes the results there too;
+  // serving batches solve a device-side count of LPs and copy only those
+  const bool mirror = mirrors(ctx, B);
+  auto at = [&](const void* d) -> void* {
+    return mirror ? B->h_res + ((const char*)d - (const char*)B->out.status) : nullptr;
+  };
+  B->chk.hi32 = (int32_t*)at(B->out.status);
+  B->chk.hf64 = (double*)at(B->out.obj);
+  B->chk.hx = (double*)at(B->out.x);
+  B->chk.hbasis = (int32_t*)at(B->out.basis);
+  B->chk.hn = B->count;
 
   if (timing) HIPCHK(ctx, hipEventRecord(B->ev[0], st));
   // one launch clears the fallback flags and every bin's queues and counts (a launch of its
@@ -906,18 +925,23 @@ int blpg_batch_solve(blpg_ctx* ctx, blpg_batch* B) {
   // where the same copies enqueued on the bins' streams took 4.3 ms (203 MB, overlapped
   // with the earlier bins' kernels).
   const int g = 0;
+  const bool mirror = mirrors(ctx, B);
+  B->mirrored = false;
   if (!ctx->opt.use_graph || B->dirty) {
     const int rc = enqueue_solve(ctx, B, true, B->dirty);
     if (!rc) B->dirty = false;
+    B->mirrored = !rc && mirror;
     return rc;
   }
   // hipGraph path: the whole sequence (clears, warm-start network, every bin's solve /
   // check / fallback on its stream, joins) is captured once per batch and replayed; it is
-  // captured again when options, the attached model or the context's workspaces change.
+  // captured again when options, the attached model, the context's workspaces or the host
+  // copy of the results change.
   blpg_options key = ctx->opt;
   key.use_graph = 1;
   const bool stale = !B->gexec[g] || std::memcmp(&key, &B->g_opt[g], sizeof key) != 0 ||
-                     B->g_model[g] != B->model || B->g_gen[g] != ctx->gen;
+                     B->g_model[g] != B->model || B->g_gen[g] != ctx->gen ||
+                     B->g_mirror[g] != mirror;
   if (stale) {
     drop_graph(B, g);
     int rc = plan_workspaces(ctx, B);  // allocations happen outside the capture
@@ -936,12 +960,14 @@ int blpg_batch_solve(blpg_ctx* ctx, blpg_batch* B) {
     B->g_opt[g] = key;
     B->g_model[g] = B->model;
     B->g_gen[g] = ctx->gen;
+    B->g_mirror[g] = mirror;
   }
   HIPCHK(ctx, hipEventRecord(B->ev[0], ctx->stream));
   HIPCHK(ctx, hipGraphLaunch(B->gexec[g], ctx->stream));
   HIPCHK(ctx, hipEventRecord(B->ev[kEvEnd], ctx->stream));
   B->nev = kEvEnd + 1;
   B->timed = false;
+  B->mirrored = mirror;
   return BLPG_OK;
 }
 
@@ -1048,8 +1074,9 @@ int blpg_batch_fetch(blpg_ctx* ctx, blpg_batch* B, blpg_batch_results* R) {
     B->h_res = nullptr;
     return fail(ctx, BLPG_E_NOMEM, "hipHostMalloc(%zu) for results failed", B->res_bytes);
   }
-  HIPCHK(ctx, hipMemcpyAsync(B->h_res, (char*)B->mem + B->res_off, B->res_bytes,
-                             hipMemcpyDeviceToHost, ctx->stream));
+  if (!B->mirrored)  // (else the solve's check kernels have written it)
+    HIPCHK(ctx, hipMemcpyAsync(B->h_res, (char*)B->mem + B->res_off, B->res_bytes,
+                               hipMemcpyDeviceToHost, ctx->stream));
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
   // the host span mirrors the device carve: int32 block, FP64 block, x pool, basis pool
   int32_t* i32 = (int32_t*)B->h_res;

@@ -47,6 +47,13 @@ struct Check {
   double* kkt_d;    // dual residual (relative)
   int32_t* ok;      // 1 verified, 0 failed (needs fallback), 2 not checkable (status kept)
   int32_t* fb;      // set to 1 when an FP32 result failed and went to the FP64 fallback
+  // Host copy (pinned memory) of the results, written LP by LP as the check ends them; all
+  // nullptr: not kept.  hi32 and hf64 hold the arrays of the device's block in its order.
+  double* hx = nullptr;
+  int32_t* hbasis = nullptr;
+  int32_t* hi32 = nullptr;
+  double* hf64 = nullptr;
+  int64_t hn = 0;   // LPs of the batch: the stride of the arrays in hi32 and hf64
 };
 
 constexpr int kStatusUndecided = 1;

@@ -862,18 +862,49 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
   }
   __syncthreads();
   // a verified result reports the FP64 basic solution: x_S from the refinement, 0 elsewhere
+  const bool fails = fp32_source && ok == 0 && fail_list;
+  double* xo = out.x + D.x;
+  const bool host = chk.hx && !fails;
+  double* hx = chk.hx + D.x;
   if (ok == 1 && kx >= 0) {
-    double* xo = out.x + D.x;
-    for (int j = tid; j < n; j += NT) xo[j] = 0.0;
-    __syncthreads();
-    for (int a = tid; a < kx; a += NT) xo[S[a]] = x[Srow[a]];
+    for (int j = tid; j < n; j += NT) {
+      const int q = rowof[j];
+      const double v = q >= 0 ? x[q] : 0.0;
+      xo[j] = v;
+      if (host) hx[j] = v;
+    }
+  } else if (host) {
+    for (int j = tid; j < n; j += NT) hx[j] = xo[j];
+  }
+  // The last check of an LP also writes its results to the host: the transfer then runs
+  // beside the other LPs' work (solve and fetch of 8192 LPs of 105x103: 0.88 ms, 1.05 ms
+  // with the copy of 10 MB after the solve; four bins of 1024: 1.08 and 1.18).
+  if (host) {
+    int32_t* hb = chk.hbasis + D.basis;
+    for (int i = tid; i < m; i += NT) hb[i] = basis[i];
   }
   if (tid == 0) {
     chk.ok[lp] = ok;
     chk.obj[lp] = zobj;
     chk.kkt_p[lp] = rp;
     chk.kkt_d[lp] = rd;
-    if (fp32_source && ok == 0 && fail_list) {
+    if (host) {
+      int32_t* hi = chk.hi32 + lp;
+      double* hf = chk.hf64 + lp;
+      const int64_t hn = chk.hn;
+      hi[0] = status;
+      hi[hn] = out.pivots[lp];
+      hi[2 * hn] = out.p1[lp];
+      hi[3 * hn] = out.unb[lp];
+      hi[4 * hn] = ok;
+      hi[5 * hn] = chk.fb[lp];
+      hf[0] = out.obj[lp];
+      hf[hn] = out.wfin[lp];
+      hf[2 * hn] = zobj;
+      hf[3 * hn] = rp;
+      hf[4 * hn] = rd;
+    }
+    if (fails) {
       const int pos = atomicAdd(fail_count, 1);
       fail_list[pos] = lp;
       chk.fb[lp] = 1;
@@ -887,7 +918,7 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
   // element that is tiny in exact arithmetic.  Its leaving variable is the final nonbasic
   // variable of the pivot column, and goes back to the pivot row.  Other failed results
   // restart cold (crash list cleared).
-  if (fp32_source && ok == 0 && fail_list) {
+  if (fails) {
     int32_t* bw = out.basis + D.basis;
     const int lpv = (undo_last && out.lastpiv) ? out.lastpiv[lp] : -1;
     const int pr = lpv & 0xFFFF, pc = lpv >> 16;
