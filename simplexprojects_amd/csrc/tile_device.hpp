@@ -19,18 +19,20 @@
 //   column  the TR owners of column s write it to LDS and zero it in their blocks -- barrier
 //   ratio   theta over the rows, minimum by DPP, ballot: r is wave-uniform
 //   row     the TC owners of row r write it to LDS and set it to -0.0 -- barrier
-//   update  block += (-column) (x) (row / p) with multiplier 1 for row r, whose -0.0 entries
+//   update  block += column (x) (row / -p) with multiplier -1 for row r, whose -0.0 entries
 //           become the scaled row exactly; the objective row is updated in column form
 //           too, so the next pricing runs beside the FMAs instead of after them
 // The pivot row's entry at column s is published as 1, which scales to the reciprocal; the
-// column is also published negated, with 1 at row r.  So neither the scaling nor the update
-// selects anything per element.
+// column is published twice, the second time with -1 at row r.  So neither the scaling nor
+// the update selects anything per element.
 //
 // What bounds it is the chain of one pivot (two LDS round trips and barriers, an FP64
-// division, two reductions).  FP64, one LP alone, per pivot: 1.62 us at 105x103, 2.17 at
-// 174x142, 2.80 at 205x203; with every reduction on one wavefront and its result broadcast
-// (four barriers), and the block as a C++ array, it was 3.26, 3.83 and 24.3 (spilled).
-// 1024 LPs of 105x103 take 1.10 ms against 2.27.
+// division, two reductions).  FP64, one LP alone, per pivot: 0.97 us at 27x32, 1.53 at
+// 105x103, 2.13 at 174x142, 2.61 at 205x203; with every reduction on one wavefront and its
+// result broadcast (four barriers), and the block as a C++ array, 105x103 took 3.26, 174x142
+// 3.83 and 205x203 24.3 (spilled).  1024 LPs of 105x103 take 1.05 ms against 2.27.  Of 4000
+// cycles at 105x103 the column's way through LDS takes 880, the ratio test 970, the row 140,
+// the reciprocal and the second barrier 650, pricing 670 and the update 700.
 //
 // Arithmetic and rule are those of kernel_stream.hip and the oracle, operation for
 // operation: results are bit-identical across kernels.  Replaces the reference's
@@ -95,6 +97,71 @@ __device__ __forceinline__ void blk_fma(T a, T b) {
   else if constexpr (G::W == 1) asm volatile("v_fmac_f32 v[%2], %0, %1" ::"v"(a), "v"(b), "n"(G::N));
   else asm volatile("v_fmac_f64 v[%2:%3], %0, %1" ::"v"(a), "v"(b), "n"(G::N), "n"(G::N + 1));
 }
+
+// Column l (row k) of a thread's block, CNT elements STEP apart in the registers, straight
+// to LDS at a0 (and a1, with TWO), OFF elements apart there; then the registers are set to z.
+// A register number cannot be dynamic, so the wave-uniform index x jumps into a table of
+// CASES equal-sized entries (clamped, so that it stays inside for any value), the first
+// elements NEXT apart: a tree of scalar branches, with a copy and a store per element in its
+// leaves, cost 200 cycles more for the column and as many for the row.  Pairs of elements share an instruction.  The caller waits for the stores (LDS
+// instructions in assembly are not the compiler's to count).
+template <typename T, int NV, int CASES, int CNT, int STEP, int NEXT, int OFF, bool TWO>
+__device__ __forceinline__ void blk_out(int x, unsigned a0, unsigned a1, T z) {
+  constexpr int W = (int)sizeof(T) / 4;
+  static_assert((CNT - 1) * OFF < 256, "offset0 and offset1 are eight bits");
+  constexpr int size = ((CNT + 1) / 2 * (TWO ? 2 : 1)) * 8 + 4 + CNT * 4 + 4;
+  int t;
+#define BLPG_OUT(ds2, ds1, mov, hi0, hi1)                                                   \
+  asm volatile(                                                                             \
+      "s_min_u32 %[t], %[x], %[cases] - 1\n\t"                                              \
+      "s_mul_i32 %[t], %[t], %[size]\n\t"                                                   \
+      "s_add_u32 %[t], %[t], 12\n\t"                                                        \
+      "s_getpc_b64 vcc\n\t"                                                                 \
+      "s_add_u32 vcc_lo, vcc_lo, %[t]\n\t"                                                  \
+      "s_addc_u32 vcc_hi, vcc_hi, 0\n\t"                                                    \
+      "s_setpc_b64 vcc\n\t"                                                                 \
+      ".set blpg_c, %[nv]\n\t"                                                              \
+      ".rept %[cases]\n\t"                                                                  \
+      ".set blpg_a, blpg_c\n\t"                                                             \
+      ".set blpg_o, 0\n\t"                                                                  \
+      ".rept %[cnt] / 2\n\t"                                                                \
+      ds2 " %[a0], v[blpg_a" hi0 "], v[" hi1 "] offset0:blpg_o offset1:blpg_o + %[off]\n\t" \
+      ".if %[two]\n\t"                                                                      \
+      ds2 " %[a1], v[blpg_a" hi0 "], v[" hi1 "] offset0:blpg_o offset1:blpg_o + %[off]\n\t" \
+      ".endif\n\t"                                                                          \
+      ".set blpg_a, blpg_a + 2 * %[step]\n\t"                                               \
+      ".set blpg_o, blpg_o + 2 * %[off]\n\t"                                                \
+      ".endr\n\t"                                                                           \
+      ".if %[cnt] & 1\n\t"                                                                  \
+      ds1 " %[a0], v[blpg_a" hi0 "] offset:%[bytes] * blpg_o\n\t"                           \
+      ".if %[two]\n\t"                                                                      \
+      ds1 " %[a1], v[blpg_a" hi0 "] offset:%[bytes] * blpg_o\n\t"                           \
+      ".endif\n\t"                                                                          \
+      ".endif\n\t"                                                                          \
+      "s_nop 1\n\t"                                                                         \
+      ".set blpg_a, blpg_c\n\t"                                                             \
+      ".rept %[cnt]\n\t"                                                                    \
+      mov " v[blpg_a" hi0 "], %[z]\n\t"                                                     \
+      ".set blpg_a, blpg_a + %[step]\n\t"                                                   \
+      ".endr\n\t"                                                                           \
+      "s_branch Lout%=\n\t"                                                                 \
+      ".set blpg_c, blpg_c + %[next]\n\t"                                                   \
+      ".endr\n"                                                                             \
+      "Lout%=:"                                                                             \
+      : [t] "=&s"(t)                                                                        \
+      : [x] "s"(x), [a0] "v"(a0), [a1] "v"(a1), [z] "v"(z), [nv] "n"(NV), [cases] "n"(CASES), \
+        [cnt] "n"(CNT), [step] "n"(W * STEP), [next] "n"(W * NEXT), [off] "n"(OFF),         \
+        [two] "n"(TWO ? 1 : 0), [size] "n"(size), [bytes] "n"(4 * W)                        \
+      : "vcc", "scc", "memory")
+  if constexpr (W == 2) BLPG_OUT("ds_write2_b64", "ds_write_b64", "v_mov_b64", ":blpg_a + 1", "blpg_a + %[step]:blpg_a + %[step] + 1");
+  else BLPG_OUT("ds_write2_b32", "ds_write_b32", "v_mov_b32", "", "blpg_a + %[step]");
+#undef BLPG_OUT
+}
+// the LDS address of a pointer into LDS, and the wait for blk_out's stores
+__device__ __forceinline__ unsigned lds_addr(const void* p) {
+  return (unsigned)(size_t)(__attribute__((address_space(3))) const char*)p;
+}
+__device__ __forceinline__ void lds_settle() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
 // compile-time loop: f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>)
 template <class F, int... I>
@@ -224,6 +291,8 @@ struct TileTab {
   static constexpr int NG = (CCAP + 63) / 64, CB = 64 * NG;  // column form
   static_assert(TC <= 32 && 64 % TC == 0, "whole rows of threads per wavefront");
   static constexpr bool kEngine = true;
+  // part of the block lies in accumulation registers (which blk_out does not address)
+  static constexpr bool kAcc = NV + (int)sizeof(T) / 4 * RPT * CPT > 256;
 
   static constexpr int el(int k, int l) { return k * CPT + l; }
   T orw[NG];      // objective row orow_in, column form (kept by engine; -1: not loaded)
@@ -237,7 +306,7 @@ struct TileTab {
   int col_ready;  // column published and zeroed (-1: none)
   int cph, rph;   // buffer phases
   T* colbuf;      // 2 x RB: published column, read in row form
-  T* colupd;      // 2 x RB: the update's multipliers (the column negated, 1 at the pivot row)
+  T* colupd;      // 2 x RB: the update's multipliers (the column, -1 at the pivot row)
   T* rhsbuf;      // RB: right-hand side, rewritten by its owners after every update
   T* rowbuf;      // 2 x CB: published row
   int* bs;        // BC: basic / nonbasic variables and the column of each nonbasic variable,
@@ -403,17 +472,23 @@ struct TileTab {
     cph ^= 1;
     T* cb = colbuf + cph * RB;
     T* cu = colupd + cph * RB;
-    dispatch<0, CPT>(ls, [&](auto l) {
+    if constexpr (ZERO && !kAcc) {
       if (gc == gcs)
-        unroll<RPT>([&](auto k) {
-          const T x = get_el<el(k, l)>();
-          cb[row_of(k)] = x;
-          if constexpr (ZERO) {
-            cu[row_of(k)] = -x;
-            set_el<el(k, l)>(T(0));
-          }
-        });
-    });
+        blk_out<T, NV, CPT, RPT, CPT, 1, TR, true>(ls, lds_addr(cb + gr), lds_addr(cu + gr), T(0));
+      lds_settle();
+    } else {
+      dispatch<0, CPT>(ls, [&](auto l) {
+        if (gc == gcs)
+          unroll<RPT>([&](auto k) {
+            const T x = get_el<el(k, l)>();
+            cb[row_of(k)] = x;
+            if constexpr (ZERO) {
+              cu[row_of(k)] = x;
+              set_el<el(k, l)>(T(0));
+            }
+          });
+      });
+    }
     __syncthreads();
 #pragma unroll
     for (int p = 0; p < RP; ++p) {
@@ -429,7 +504,7 @@ struct TileTab {
     const int ls = s / TC, gcs = s - ls * TC;
     const T* cu = colupd + cph * RB;
     dispatch<0, CPT>(ls, [&](auto l) {
-      if (gc == gcs) unroll<RPT>([&](auto k) { set_el<el(k, l)>(-cu[row_of(k)]); });
+      if (gc == gcs) unroll<RPT>([&](auto k) { set_el<el(k, l)>(cu[row_of(k)]); });
     });
     col_ready = -1;
   }
@@ -441,13 +516,18 @@ struct TileTab {
     const int kr = r / TR, grr = r - kr * TR;
     rph ^= 1;
     T* rb = rowbuf + rph * CB;
-    dispatch<0, RPT>(kr, [&](auto k) {
+    if constexpr (CLEAR && !kAcc) {
       if (gr == grr)
-        unroll<CPT>([&](auto l) {
-          rb[col_of(l)] = get_el<el(k, l)>();
-          if constexpr (CLEAR) set_el<el(k, l)>(T(-0.0));
-        });
-    });
+        blk_out<T, NV, RPT, CPT, 1, CPT, TC, false>(kr, lds_addr(rb + gc), 0, T(-0.0));
+    } else {
+      dispatch<0, RPT>(kr, [&](auto k) {
+        if (gr == grr)
+          unroll<CPT>([&](auto l) {
+            rb[col_of(l)] = get_el<el(k, l)>();
+            if constexpr (CLEAR) set_el<el(k, l)>(T(-0.0));
+          });
+      });
+    }
     if constexpr (CLEAR) {
       // (same wavefront, after the row's own stores)
       if (gr == grr && gc == 0) rb[s] = T(1);
@@ -579,14 +659,15 @@ struct TileTab {
         }
         rb = write_row<true>(r, s);
         cu = colupd + cph * RB;
-        if (tid == 0) colupd[cph * RB + r] = T(1);
-        rp = T(1) / pick(acol, r);
+        if (tid == 0) colupd[cph * RB + r] = T(-1);
+        rp = T(-1) / pick(acol, r);
         const int e = pick(nbv, s), lv = pick(bsr, r);  // entering, leaving variable
 #pragma unroll
         for (int p = 0; p < RP; ++p) bsr[p] = (lane + 64 * p == r) ? e : bsr[p];
 #pragma unroll
         for (int g = 0; g < NG; ++g) nbv[g] = (lane + 64 * g == s) ? lv : nbv[g];
         if (fast) c0 = pick(orw, s);
+        if constexpr (!kAcc) lds_settle();
         __syncthreads();
       }
       int sn = -1;
@@ -595,7 +676,7 @@ struct TileTab {
         for (int g = 0; g < NG; ++g) {
           const int j = lane + 64 * g;
           const T pr = rb[j] * rp;
-          const T d = fma_t(-c0, pr, j == s ? T(0) : orw[g]);
+          const T d = fma_t(c0, pr, j == s ? T(0) : orw[g]);
           orw[g] = j < C ? d : T(0);
         }
         sn = price(o.eps_d);
