@@ -549,6 +549,39 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
                             : q[0] + q[1]);
       }
     };
+    // The same from global memory (blocks too large for the last tier): emit(a, sum over the
+    // rows p of M[p ld + col(a)] v[p]).  Threads of neighbouring a read neighbouring entries
+    // of a row; up to eight threads per column share its rows, eight loads in flight each (sixteen spill).  1024 LPs of 205x203, whose
+    // blocks mostly exceed LDS: check 2.7 -> 1.26 ms against one thread per column.
+    auto colsum_mem = [&](const auto* M, int64_t ld, const double* v, int cnt, auto&& col, auto&& emit) {
+      const int sh = cnt == 0 || 2 * cnt > NT ? 0 : 4 * cnt > NT ? 1 : 8 * cnt > NT ? 2 : 3;
+      const int per = 1 << sh;
+      const int ta = sh ? tid % cnt : tid, tp = sh ? tid / cnt : 0;
+      if (tp < per)
+        for (int a = ta; a < cnt; a += sh ? cnt : NT) {
+          const auto* Mc = M + col(a);
+          double t[4] = {0, 0, 0, 0};
+#pragma unroll 1
+          for (int p = tp; p < m; p += 8 * per) {
+            double e[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) e[u] = (double)Mc[ld * min(p + u * per, m - 1)];
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+              if (p + u * per < m) t[u % 4] = fma(e[u], v[p + u * per], t[u % 4]);
+          }
+          const double q = (t[0] + t[1]) + (t[2] + t[3]);
+          if (sh) part[tp * cnt + a] = q;
+          else emit(a, q);
+        }
+      if (!sh) return;
+      __syncthreads();
+      if (tid < cnt) {
+        double q = part[tid];
+        for (int i = 1; i < per; ++i) q += part[i * cnt + tid];
+        emit(tid, q);
+      }
+    };
     // f(j, sum over rows of A[p][j] w[p]) for every structural column j: G threads per column,
     // 16 loads in flight each; their sums meet in LDS
     auto a_columns = [&](auto&& f) {
@@ -635,21 +668,12 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
             rl = fmax(rl, fabs(sum));
           });
         } else {
-          for (int a = tid; a < k; a += NT) {
-            double s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-            int p = 0;
-            const int v = S[a];
-            for (; p + 4 <= m; p += 4) {
-              s0 = fma(sg(p) * A[(int64_t)p * n + v], y[p], s0);
-              s1 = fma(sg(p + 1) * A[(int64_t)(p + 1) * n + v], y[p + 1], s1);
-              s2 = fma(sg(p + 2) * A[(int64_t)(p + 2) * n + v], y[p + 2], s2);
-              s3 = fma(sg(p + 3) * A[(int64_t)(p + 3) * n + v], y[p + 3], s3);
-            }
-            for (; p < m; ++p) s0 = fma(sg(p) * A[(int64_t)p * n + v], y[p], s0);
-            const double sum = (s0 + s1) + (s2 + s3);
+          for (int p = tid; p < m; p += NT) w[p] = sg(p) * y[p];
+          __syncthreads();
+          colsum_mem(A, n, w, k, [&](int a) { return S[a]; }, [&](int a, double sum) {
             rho[Srow[a]] = -sum;
             rl = fmax(rl, fabs(sum));
-          }
+          });
         }
         for (int p = tid; p < m; p += NT) {
           const int q = rowof[n + p];
@@ -668,19 +692,8 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
         if (staged) {
           colsum(TB, rho, kq, [&](int a, double sum) { y[Pn[a]] += sum; });
         } else {
-          for (int a = tid; a < kq; a += NT) {
-            double s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-            int i = 0;
-            const int j = Pcol[a];
-            for (; i + 4 <= m; i += 4) {
-              s0 = fma((double)T[(int64_t)(2 + i) * C + j], rho[i], s0);
-              s1 = fma((double)T[(int64_t)(3 + i) * C + j], rho[i + 1], s1);
-              s2 = fma((double)T[(int64_t)(4 + i) * C + j], rho[i + 2], s2);
-              s3 = fma((double)T[(int64_t)(5 + i) * C + j], rho[i + 3], s3);
-            }
-            for (; i < m; ++i) s0 = fma((double)T[(int64_t)(2 + i) * C + j], rho[i], s0);
-            y[Pn[a]] += (s0 + s1) + (s2 + s3);
-          }
+          colsum_mem(T + 2 * (int64_t)C, C, rho, kq, [&](int a) { return Pcol[a]; },
+                     [&](int a, double sum) { y[Pn[a]] += sum; });
         }
         for (int p = tid; p < m; p += NT) {
           const int q = rowof[n + p];
@@ -744,21 +757,13 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
               rl = fmax(rl, fabs(val));
             });
           } else {
-            for (int a = tid; a < k; a += NT) {
-              double s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-              int p = 0;
-              const int v = S[a];
-              for (; p + 4 <= m; p += 4) {
-                s0 = fma(sg(p) * A[(int64_t)p * n + v], y[p], s0);
-                s1 = fma(sg(p + 1) * A[(int64_t)(p + 1) * n + v], y[p + 1], s1);
-                s2 = fma(sg(p + 2) * A[(int64_t)(p + 2) * n + v], y[p + 2], s2);
-                s3 = fma(sg(p + 3) * A[(int64_t)(p + 3) * n + v], y[p + 3], s3);
-              }
-              for (; p < m; ++p) s0 = fma(sg(p) * A[(int64_t)p * n + v], y[p], s0);
-              const double val = cS[a] - ((s0 + s1) + (s2 + s3));
+            for (int p = tid; p < m; p += NT) w[p] = sg(p) * y[p];
+            __syncthreads();
+            colsum_mem(A, n, w, k, [&](int a) { return S[a]; }, [&](int a, double sum) {
+              const double val = cS[a] - sum;
               rho[Srow[a]] = val;
               rl = fmax(rl, fabs(val));
-            }
+            });
           }
           for (int p = tid; p < m; p += NT) {
             const int q = rowof[n + p];
@@ -776,19 +781,8 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
           if (staged) {
             colsum(TB, rho, k, [&](int a, double sum) { y[Pn[a]] += sum; });
           } else {
-            for (int a = tid; a < k; a += NT) {
-              double s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-              int i = 0;
-              const int j = Pcol[a];
-              for (; i + 4 <= m; i += 4) {
-                s0 = fma((double)T[(int64_t)(2 + i) * C + j], rho[i], s0);
-                s1 = fma((double)T[(int64_t)(3 + i) * C + j], rho[i + 1], s1);
-                s2 = fma((double)T[(int64_t)(4 + i) * C + j], rho[i + 2], s2);
-                s3 = fma((double)T[(int64_t)(5 + i) * C + j], rho[i + 3], s3);
-              }
-              for (; i < m; ++i) s0 = fma((double)T[(int64_t)(2 + i) * C + j], rho[i], s0);
-              y[Pn[a]] += (s0 + s1) + (s2 + s3);
-            }
+            colsum_mem(T + 2 * (int64_t)C, C, rho, k, [&](int a) { return Pcol[a]; },
+                       [&](int a, double sum) { y[Pn[a]] += sum; });
           }
           for (int p = tid; p < m; p += NT) {
             const int q = rowof[n + p];
