@@ -232,6 +232,31 @@ def _lp_struct(lp: LP) -> _LP:
     return s
 
 
+# blpg_lp and blpg_result with plain integers for pointers, to be filled a column at a time
+_LP_DT = np.dtype([("m", np.int32), ("n", np.int32), ("A", np.uintp), ("b", np.uintp),
+                   ("c", np.uintp), ("sense", np.uintp), ("family", np.int32),
+                   ("warm_basis", np.uintp)], align=True)
+_RESULT_DT = np.dtype([("status", np.int32), ("pivots", np.int32), ("phase1_pivots", np.int32),
+                       ("fallback_used", np.int32), ("objective", np.float64),
+                       ("kkt_primal", np.float64), ("kkt_dual", np.float64), ("x", np.uintp),
+                       ("basis", np.uintp)], align=True)
+assert _LP_DT.itemsize == C.sizeof(_LP) and _RESULT_DT.itemsize == C.sizeof(_Result)
+
+
+def _addr(a: Optional[np.ndarray]) -> int:
+    return 0 if a is None else a.__array_interface__["data"][0]
+
+
+def _lp_array(lps: Sequence[LP]):
+    """blpg_lp array of the LPs (the LPs must outlive its use).  One record array instead of
+    a ctypes structure per LP, whose pointer fields cost 2 us each."""
+    if not lps:
+        return (_LP * 0)()
+    rows = [(lp.m, lp.n, _addr(lp.A), _addr(lp.b), _addr(lp.c), _addr(lp.sense), lp.family,
+             _addr(lp.warm_basis)) for lp in lps]
+    return (_LP * len(rows)).from_buffer(np.array(rows, dtype=_LP_DT))
+
+
 def gen_config(config: int, seed: int, m: int, n: int, count: int, shape_idx: int = 0,
                first: int = 0, batch_count: Optional[int] = None) -> list[LP]:
     """Seeded synthetic LPs (host generator in libblpg; see csrc/gen.cpp)."""
@@ -272,26 +297,26 @@ class Results:
 
 
 def _alloc_results(lps: Sequence[LP]):
+    """(blpg_result array, xs, bases): the vectors are slices of two pools, so that one
+    address serves them all."""
     k = len(lps)
-    res = (_Result * k)()
-    xs = [np.zeros(lp.n) for lp in lps]
-    bs = [np.zeros(lp.m, dtype=np.int32) for lp in lps]
-    for i in range(k):
-        res[i].x = _dp(xs[i])
-        res[i].basis = bs[i].ctypes.data_as(C.POINTER(C.c_int32))
-    return res, xs, bs
+    if k == 0:
+        return (_Result * 0)(), [], []
+    xo = np.concatenate([[0], np.cumsum([lp.n for lp in lps])])
+    bo = np.concatenate([[0], np.cumsum([lp.m for lp in lps])])
+    xp, bp = np.zeros(xo[-1]), np.zeros(bo[-1], dtype=np.int32)
+    rec = np.zeros(k, dtype=_RESULT_DT)
+    rec["x"] = _addr(xp) + 8 * xo[:-1].astype(np.uintp)
+    rec["basis"] = _addr(bp) + 4 * bo[:-1].astype(np.uintp)
+    cut = lambda pool, o: [pool[i:j] for i, j in zip(o[:-1].tolist(), o[1:].tolist())]
+    return (_Result * k).from_buffer(rec), cut(xp, xo), cut(bp, bo)
 
 
 def _collect(res, xs, bs) -> Results:
     k = len(xs)
     # view the result records through a pointer-free mirror of blpg_result
-    dt = np.dtype([("status", np.int32), ("pivots", np.int32), ("phase1_pivots", np.int32),
-                   ("fallback_used", np.int32), ("objective", np.float64),
-                   ("kkt_primal", np.float64), ("kkt_dual", np.float64), ("x", np.uintp),
-                   ("basis", np.uintp)])
-    assert dt.itemsize == C.sizeof(_Result)
     arr = np.frombuffer((C.c_char * (C.sizeof(_Result) * k)).from_address(C.addressof(res)),
-                        dtype=dt, count=k) if k else np.zeros(0, dtype=dt)
+                        dtype=_RESULT_DT, count=k) if k else np.zeros(0, dtype=_RESULT_DT)
     return Results(arr["status"].copy(), arr["pivots"].copy(), arr["phase1_pivots"].copy(),
                    arr["fallback_used"].copy(), arr["objective"].copy(),
                    arr["kkt_primal"].copy(), arr["kkt_dual"].copy(), xs, bs)
@@ -303,7 +328,7 @@ class Batch:
     def __init__(self, solver: "Solver", lps: Sequence[LP]):
         self.solver = solver
         self.lps = list(lps)
-        arr = (_LP * len(self.lps))(*[_lp_struct(lp) for lp in self.lps])
+        arr = _lp_array(self.lps)
         h = C.c_void_p()
         solver._check(solver.lib.blpg_batch_upload(solver.ctx, arr, len(self.lps), C.byref(h)))
         self.h = h
@@ -315,7 +340,7 @@ class Batch:
         """New LPs of the same shapes into the batch's pinned staging (host work); the next
         solve() copies them to the device before its kernels."""
         lps = list(lps)
-        arr = (_LP * len(lps))(*[_lp_struct(lp) for lp in lps])
+        arr = _lp_array(lps)
         self.solver._check(self.solver.lib.blpg_batch_repack(self.solver.ctx, self.h, arr,
                                                              len(lps)))
         self.lps = lps
@@ -424,7 +449,7 @@ class Solver:
 
     def solve(self, lps: Sequence[LP]) -> Results:
         lps = list(lps)
-        arr = (_LP * len(lps))(*[_lp_struct(lp) for lp in lps])
+        arr = _lp_array(lps)
         res, xs, bs = _alloc_results(lps)
         self._check(self.lib.blpg_solve_batch(self.ctx, arr, len(lps), res))
         return _collect(res, xs, bs)
@@ -451,7 +476,7 @@ class Solver:
         shape's check plan (kernel 0 rows: param 1 skips the first check tier); returns the
         tuning table as (precision, m, n, kernel, param, ms) tuples."""
         lps = list(lps)
-        arr = (_LP * len(lps))(*[_lp_struct(lp) for lp in lps])
+        arr = _lp_array(lps)
         self._check(self.lib.blpg_autotune(self.ctx, arr, len(lps), reps))
         return self.tune_table()
 
@@ -515,7 +540,7 @@ class WarmStart:
 
     def _lps(self, lps):
         lps = list(lps)
-        return lps, (_LP * len(lps))(*[_lp_struct(lp) for lp in lps])
+        return lps, _lp_array(lps)
 
     def train(self, lps: Sequence[LP], bases: Sequence[np.ndarray]) -> np.ndarray:
         lps, arr = self._lps(lps)
@@ -636,7 +661,7 @@ class Server:
     def replay(self, lps: Sequence[LP], arrival_us: np.ndarray):
         """Submit lps[k] at arrival_us[k] (from now) and wait for all; per-LP results."""
         lps = list(lps)
-        arr = (_LP * len(lps))(*[_lp_struct(lp) for lp in lps])
+        arr = _lp_array(lps)
         t = np.ascontiguousarray(arrival_us, dtype=np.float64)
         out = (_ServerResult * len(lps))()
         rc = self.solver.lib.blpg_server_replay(self.h, arr, _dp(t), len(lps), out)

@@ -8,12 +8,14 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
 #include <map>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/blpg/blpg.h"
@@ -38,9 +40,16 @@ void resolve(const blpg_options& o, double& eps_d, double& eps_p, double& tol, d
 int bland_after(const blpg_options& o) { return o.bland_after > 0 ? o.bland_after : 50; }
 
 bool finite_all(const double* p, int64_t n) {
-  for (int64_t i = 0; i < n; ++i)
-    if (!std::isfinite(p[i])) return false;
-  return true;
+  // x - x is +0.0 for every finite x and NaN for the others; without a branch per element
+  // the loop runs in vector registers
+  uint64_t acc = 0;
+  for (int64_t i = 0; i < n; ++i) {
+    const double d = p[i] - p[i];
+    uint64_t u;
+    std::memcpy(&u, &d, sizeof u);
+    acc |= u;
+  }
+  return acc == 0;
 }
 
 int grow(blpg_ctx* ctx, DevBuf& b, size_t bytes) {
@@ -345,29 +354,38 @@ int blpg_batch_upload(blpg_ctx* ctx, const blpg_lp* lps, int64_t count, blpg_bat
   //      device on the bin's own stream just before its kernel; arrays several bins read
   //      form a common range in front, copied first. ----
   {
-    std::map<SrcKey, int> key_bin;  // the one bin reading the array, or -1 (several)
+    // one lookup per array; the LPs then hold on to what it found
+    struct Source { int bin; int64_t off; };  // bin: the one reading the array, -1: several
+    struct Hash {
+      size_t operator()(const SrcKey& k) const {
+        return ((uintptr_t)k.first ^ ((uint64_t)k.second << 20)) * 0x9E3779B97F4A7C15ull >> 16;
+      }
+    };
+    std::unordered_map<SrcKey, Source, Hash> sources(3 * (size_t)count);
+    std::vector<std::array<Source*, 3>> src(count);
+    auto arrays = [&](int64_t k) {
+      const blpg_lp& L = lps[k];
+      return std::array<SrcKey, 3>{SrcKey(L.A, (int64_t)L.m * L.n), SrcKey(L.b, L.m), SrcKey(L.c, L.n)};
+    };
     for (int bi = 0; bi < (int)B->bins.size(); ++bi)
       for (int32_t k : B->bins[bi].ids) {
-        const blpg_lp& L = lps[k];
-        for (const SrcKey& key : {SrcKey(L.A, (int64_t)L.m * L.n), SrcKey(L.b, L.m), SrcKey(L.c, L.n)}) {
-          auto it = key_bin.find(key);
-          if (it == key_bin.end()) key_bin[key] = bi;
-          else if (it->second != bi) it->second = -1;
+        const auto keys = arrays(k);
+        for (int i = 0; i < 3; ++i) {
+          Source& s = sources.emplace(keys[i], Source{bi, -1}).first->second;
+          if (s.bin != bi) s.bin = -1;
+          src[k][i] = &s;
         }
       }
     int64_t bad = -1;
-    auto place = [&](const double* p, int64_t len, int64_t k) {
-      const SrcKey key(p, len);
-      if (B->pool_off.count(key)) return;
-      if (bad < 0 && !finite_all(p, len)) bad = k;
-      B->pool_off[key] = B->pool_elems;
-      B->pool_elems += (len + 7) & ~7ll;
-    };
     auto place_lp = [&](int64_t k, int want_bin) {
-      const blpg_lp& L = lps[k];
-      if (key_bin[SrcKey(L.A, (int64_t)L.m * L.n)] == want_bin) place(L.A, (int64_t)L.m * L.n, k);
-      if (key_bin[SrcKey(L.b, L.m)] == want_bin) place(L.b, L.m, k);
-      if (key_bin[SrcKey(L.c, L.n)] == want_bin) place(L.c, L.n, k);
+      const auto keys = arrays(k);
+      for (int i = 0; i < 3; ++i) {
+        Source& s = *src[k][i];
+        if (s.bin != want_bin || s.off >= 0) continue;
+        if (bad < 0 && !finite_all((const double*)keys[i].first, keys[i].second)) bad = k;
+        s.off = B->pool_elems;
+        B->pool_elems += (keys[i].second + 7) & ~7ll;
+      }
     };
     for (int64_t k = 0; k < count; ++k) place_lp(k, -1);
     B->common_elems = B->pool_elems;
@@ -384,9 +402,9 @@ int blpg_batch_upload(blpg_ctx* ctx, const blpg_lp* lps, int64_t count, blpg_bat
     for (int64_t k = 0; k < count; ++k) {
       const blpg_lp& L = lps[k];
       LpDesc& d = B->desc[k];
-      d.a = B->pool_off[SrcKey(L.A, (int64_t)L.m * L.n)];
-      d.b = B->pool_off[SrcKey(L.b, L.m)];
-      d.c = B->pool_off[SrcKey(L.c, L.n)];
+      d.a = src[k][0]->off;
+      d.b = src[k][1]->off;
+      d.c = src[k][2]->off;
       if (L.sense) {
         const SrcKey key(L.sense, L.m);
         auto it = B->spool_off.find(key);

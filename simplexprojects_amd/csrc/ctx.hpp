@@ -78,7 +78,7 @@ struct blpg_batch {
   std::vector<blpg::LpDesc> desc;
   int64_t pool_elems = 0, spool_elems = 0, x_elems = 0, basis_elems = 0, tab_elems = 0;
   int64_t common_elems = 0;  // pool[0, common_elems): arrays read by several bins
-  std::map<blpg::SrcKey, int64_t> pool_off, spool_off;  // where each distinct array lives
+  std::map<blpg::SrcKey, int64_t> spool_off;  // where each distinct sense array lives
   char* h_stage = nullptr;   // pinned host image of desc | pool | sense pool | int32 init
   size_t stage_bytes = 0, o_pool = 0, o_spool = 0;
   bool dirty = false;        // staging newer than the device copy: the next solve copies it
