@@ -657,9 +657,15 @@ struct WaveTab {
       z0 = fma_t(-c0, prow0, z0);
       z1 = fma_t(-c1, prow0, z1);
       // tiles in the matrix pipe, the next column's pricing between them (a step of the
-      // minimum after every few matrix instructions, which it would otherwise wait for)
+      // minimum after every few matrix instructions, which it would otherwise wait for).
+      // Instructions issue in order, so what stands behind the last matrix instruction waits
+      // for all of them.  With several wavefronts the bookkeeping and the end of the pricing
+      // go in between: 205x203 per pivot 1.86 -> 1.83 us, 174x142 and 250x249 2% less too (with
+      // one wavefront it changed nothing at 105x103 and cost 1% at 74x83).
       float pk = price_key(d);
       constexpr int NM = CH * G;
+      static_assert(NW == 1 || NM >= 8);
+      int sn = -1;
       acc_ready();
       unroll<NM>([&](auto u) {
         constexpr int ch = u / G, g = u % G;
@@ -670,13 +676,25 @@ struct WaveTab {
           min_step<u < 6 ? (int)u : 0>(pk);
           __builtin_amdgcn_sched_barrier(0);
         }
+        if constexpr (NW > 1 && u == 6) {
+#pragma unroll
+          for (int p = 0; p < RP; ++p) asm volatile("" : "+v"(rhs[p]), "+v"(bsr[p]));
+#pragma unroll
+          for (int j = 0; j < NG; ++j) asm volatile("" : "+v"(row0[j]), "+v"(row1[j]), "+v"(nbv[j]));
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (NW > 1 && u == 7) {
+          sn = price_end(d, pk, rdlane(pk, 63));
+          asm volatile("" ::"s"(sn));
+          __builtin_amdgcn_sched_barrier(0);
+        }
       });
       if constexpr (NM < 6) unroll<6>([&](auto u) { if constexpr (u >= NM) min_step<(int)u>(pk); });
       last = keep_last ? r | (s << 16) : -1;
       col_ready = -1;
       ++it;
       if (!fast || it >= maxit || deg >= o.bland_after) return kEngDone;
-      const int sn = price_end(d, pk, rdlane(pk, 63));
+      if constexpr (NW == 1) sn = price_end(d, pk, rdlane(pk, 63));
       if (sn < 0) return kEngDone;
       s = sn;
       r = -1;
