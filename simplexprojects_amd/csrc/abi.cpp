@@ -178,7 +178,7 @@ int blpg::set_free_error(int code, const char* fmt, ...) {
 void blpg::warm_route(blpg_batch* B) {
   for (size_t i = 0; i < B->bins.size(); ++i) {
     Bin& b = B->bins[i];
-    if (b.kernel != BLPG_KERNEL_WAVE) continue;
+    if (b.kernel != BLPG_KERNEL_WAVE && !b.many) continue;
     const int tv = Tuner::best_tile(b.rcap - 2, b.ccap - 2, B->precision);
     if (tv < 0) continue;
     b.kernel = BLPG_KERNEL_TILE;
@@ -308,17 +308,39 @@ int blpg_batch_upload(blpg_ctx* ctx, const blpg_lp* lps, int64_t count, blpg_bat
   std::vector<Route> routes(count);
   for (int64_t k = 0; k < count; ++k)
     routes[k] = ctx->tuner.route(B->desc[k].m, B->desc[k].n, ctx->opt.precision, ctx->opt.kernel);
+  bool any_warm = false;
+  for (int64_t k = 0; k < count; ++k) any_warm |= lps[k].warm_basis != nullptr;
   auto bin_key = [](const Route& r) -> long {
     if (r.kernel == BLPG_KERNEL_TILE) return 1000000L + r.variant;
     if (r.kernel == BLPG_KERNEL_WAVE) return 4000000L + r.variant;
     if (r.kernel == BLPG_KERNEL_STREAM) return 2000000L + r.nt;
     return 3000000L + (long)r.nt * 100000L + r.bin;  // LDS: per size class
   };
+  // statically routed shapes of a bin with many LPs may have a better instance (not with
+  // warm lists: those need the block crash)
+  std::vector<Route> chosen = routes;
+  std::vector<uint8_t> many(count, 0);
+  if (ctx->opt.kernel == BLPG_KERNEL_AUTO && !any_warm) {
+    auto free_route = [&](int64_t k) {
+      return !ctx->tuner.has_preference(ctx->opt.precision, B->desc[k].m, B->desc[k].n);
+    };
+    std::map<long, int64_t> fit;  // LPs of a bin that its other instance holds
+    const int cus = ctx->props.multiProcessorCount;
+    for (int64_t k = 0; k < count; ++k) {
+      Route r = routes[k];
+      if (free_route(k) && Tuner::for_many(r, B->desc[k].m, B->desc[k].n, ctx->opt.precision, INT64_MAX, cus))
+        ++fit[bin_key(routes[k])];
+    }
+    if (!fit.empty())
+      for (int64_t k = 0; k < count; ++k)
+        many[k] = free_route(k) && Tuner::for_many(chosen[k], B->desc[k].m, B->desc[k].n, ctx->opt.precision,
+                                                   fit[bin_key(routes[k])], cus);
+  }
   for (int pass = 0; pass < 2; ++pass) {
     std::map<long, int> binof;
     B->bins.clear();
     for (int64_t k = 0; k < count; ++k) {
-      const Route& r = routes[k];
+      const Route& r = chosen[k];
       const long key = bin_key(r);
       auto it = binof.find(key);
       int bi;
@@ -329,6 +351,7 @@ int blpg_batch_upload(blpg_ctx* ctx, const blpg_lp* lps, int64_t count, blpg_bat
         b.kernel = r.kernel;
         b.variant = r.variant;
         b.nt = r.nt;
+        b.many = many[k] != 0;
         B->bins.push_back(b);
       } else {
         bi = it->second;
@@ -339,7 +362,9 @@ int blpg_batch_upload(blpg_ctx* ctx, const blpg_lp* lps, int64_t count, blpg_bat
       b.ccap = std::max(b.ccap, B->desc[k].n + 2);
     }
     if (B->bins.size() <= 16) break;
-    for (auto& r : routes)
+    chosen = routes;
+    std::fill(many.begin(), many.end(), 0);
+    for (auto& r : chosen)
       if (r.kernel == BLPG_KERNEL_LDS) r.kernel = BLPG_KERNEL_STREAM;
   }
   if (B->bins.size() > 16) {
@@ -439,8 +464,6 @@ int blpg_batch_upload(blpg_ctx* ctx, const blpg_lp* lps, int64_t count, blpg_bat
   const size_t o_basis = off; off += al(sizeof(int32_t) * B->basis_elems);
   const size_t o_tab = off; off += al(8 * (size_t)B->tab_elems);
   const size_t o_cnt = off; off += al(sizeof(int32_t) * 256);
-  bool any_warm = false;
-  for (int64_t k = 0; k < count; ++k) any_warm |= lps[k].warm_basis != nullptr;
   const size_t o_warm = off;
   if (any_warm) off += al(sizeof(int32_t) * B->basis_elems);
   B->mem_bytes = off;
@@ -568,6 +591,17 @@ void blpg_batch_free(blpg_ctx* ctx, blpg_batch* B) {
   delete B;
 }
 
+// FP64 route of a bin's shapes by size alone (its instance: `f`)
+static void route64(blpg_ctx* ctx, const Bin& b, Bin& f) {
+  f.rcap = b.rcap; f.ccap = b.ccap; f.nt = Tuner::stream_threads(b.rcap - 2, b.ccap - 2);
+  const int tv = Tuner::best_tile(b.rcap - 2, b.ccap - 2, BLPG_FP64);
+  if (tv >= 0) { f.kernel = BLPG_KERNEL_TILE; f.variant = tv; }
+  else if (stream_lds_bytes(BLPG_FP64, true, f.nt, f.rcap, f.ccap) <= ctx->tuner.lds_limit() &&
+           stream_max_blocks_per_cu(BLPG_FP64, true, f.nt, f.rcap, f.ccap) > 0)
+    f.kernel = BLPG_KERNEL_LDS;
+  else f.kernel = BLPG_KERNEL_STREAM;
+}
+
 // Launch plan of one size bin: kernel, persistent grid and HBM slab size.
 struct BinPlan {
   int grid = 1;
@@ -640,7 +674,7 @@ static int launch_bin(blpg_ctx* ctx, blpg_batch* B, const Bin& b, const BinPlan&
 // and the LU slabs of the check (bins run concurrently, so each gets its own region).
 struct SolvePlan {
   std::vector<BinPlan> plans, fplans;
-  std::vector<Bin> fbins;
+  std::vector<Bin> sbins, fbins;  // instances of the solve and of the FP64 re-solve (no ids)
   std::vector<size_t> ws_off, fws_off, vws_off;
   std::vector<std::vector<int>> vtiers;  // per bin: (tier, grid) pairs of the check, in order
   std::vector<int64_t> vstride;
@@ -651,7 +685,7 @@ static int plan_solve(blpg_ctx* ctx, blpg_batch* B, SolvePlan& P) {
   const int precision = ctx->opt.precision;
   const bool do_verify = ctx->opt.verify || precision == BLPG_FP32;
   const bool fp32 = precision == BLPG_FP32;
-  P.plans.assign(nb, BinPlan{}); P.fplans.assign(nb, BinPlan{}); P.fbins.assign(nb, Bin{});
+  P.plans.assign(nb, BinPlan{}); P.fplans.assign(nb, BinPlan{}); P.fbins.assign(nb, Bin{}); P.sbins.assign(nb, Bin{});
   P.ws_off.assign(nb, 0); P.fws_off.assign(nb, 0); P.vws_off.assign(nb, 0);
   P.vtiers.assign(nb, {});
   P.vstride.assign(nb, 0);
@@ -666,7 +700,14 @@ static int plan_solve(blpg_ctx* ctx, blpg_batch* B, SolvePlan& P) {
   for (int i = 0; i < nb; ++i) {
     const Bin& b = B->bins[i];
     const int64_t cnt = (int64_t)b.ids.size();
-    int rc = plan_bin(ctx, b, precision, cnt, plans[i]);
+    // a batch routed for FP32 and solved in FP64: instances that have no FP64 form give way
+    // to the FP64 route of their shapes
+    Bin& s = P.sbins[i];
+    s.kernel = b.kernel; s.variant = b.variant; s.nt = b.nt; s.rcap = b.rcap; s.ccap = b.ccap;
+    if (!fp32 && ((b.kernel == BLPG_KERNEL_WAVE && wave_max_blocks_per_cu(precision, b.variant) <= 0) ||
+                  (b.kernel == BLPG_KERNEL_TILE && tile_max_blocks_per_cu(precision, b.variant) <= 0)))
+      route64(ctx, b, s);
+    int rc = plan_bin(ctx, s, precision, cnt, plans[i]);
     if (rc) return rc;
     ws_off[i] = ws_total;
     ws_total += plans[i].ws_bytes;
@@ -692,13 +733,7 @@ static int plan_solve(blpg_ctx* ctx, blpg_batch* B, SolvePlan& P) {
     if (fp32) {
       // FP64 fallback kernel of this bin
       Bin& f = fbins[i];
-      f.rcap = b.rcap; f.ccap = b.ccap; f.nt = Tuner::stream_threads(b.rcap - 2, b.ccap - 2);
-      const int tv = Tuner::best_tile(b.rcap - 2, b.ccap - 2, BLPG_FP64);
-      if (tv >= 0) { f.kernel = BLPG_KERNEL_TILE; f.variant = tv; }
-      else if (stream_lds_bytes(BLPG_FP64, true, f.nt, f.rcap, f.ccap) <= ctx->tuner.lds_limit() &&
-               stream_max_blocks_per_cu(BLPG_FP64, true, f.nt, f.rcap, f.ccap) > 0)
-        f.kernel = BLPG_KERNEL_LDS;
-      else f.kernel = BLPG_KERNEL_STREAM;
+      route64(ctx, b, f);
       rc = plan_bin(ctx, f, BLPG_FP64, cnt, fplans[i]);
       if (rc) return rc;
       fws_off[i] = fws_total;
@@ -864,7 +899,7 @@ static int enqueue_solve(blpg_ctx* ctx, blpg_batch* B, bool timing, bool copy) {
     if (timing) HIPCHK(ctx, hipEventRecord(B->ev[1 + 4 * i], s));
     // arena batches (serving) take their LP count from the device, so one captured graph
     // serves every batch size up to the capacity
-    int rc = launch_bin(ctx, B, b, plans[i], precision, b.d_idx, cnt, B->d_count, qb,
+    int rc = launch_bin(ctx, B, P.sbins[i], plans[i], precision, b.d_idx, cnt, B->d_count, qb,
                         (char*)ctx->ws.p + ws_off[i], B->d_warm, s);
     if (rc) return rc;
     if (timing) HIPCHK(ctx, hipEventRecord(B->ev[2 + 4 * i], s));

@@ -39,6 +39,7 @@ struct Bin {
   int variant = 0;                  // tile variant
   int nt = 256;                     // stream threads
   int rcap = 0, ccap = 0;
+  bool many = false;                // instance chosen for the number of LPs (Tuner::for_many)
   std::vector<int32_t> ids;
   int32_t* d_idx = nullptr;
   int64_t pool_lo = 0, pool_hi = 0;  // the bin's own range of the input pool (elements)
@@ -157,8 +158,8 @@ int set_free_error(int code, const char* fmt, ...);
 // results of slots 0..k-1 of a batch (abi.cpp; the serving arenas use it)
 int batch_fetch_prefix(blpg_ctx* ctx, blpg_batch* B, int64_t k, blpg_batch_results* R);
 
-// Batches with warm-start lists crash in blocks in the register-tile kernel: its bins
-// routed to the column-per-lane kernel (which crashes one target at a time) move to the
+// Batches with warm-start lists crash in blocks in the register-block kernel: bins
+// routed to the accumulator kernel (which crashes one target at a time) move to the
 // tile variant that holds their shape (abi.cpp).
 void warm_route(blpg_batch* B);
 

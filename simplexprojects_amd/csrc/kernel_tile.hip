@@ -7,6 +7,7 @@ namespace blpg {
   BLPG_TILE_KERNEL(k_tile_f32_##id, float, nw, tc, rpt, cpt, vr32, 1, false)           \
   BLPG_TILE_KERNEL(k_tile_f32w_##id, float, nw, tc, rpt, cpt, vr32w, 1, b32 != 0)
 BLPG_TILE_VARIANTS(X)
+BLPG_TILE_VARIANTS_F32(X)
 #undef X
 
 // warm: the batch carries warm-start lists (block crash where the variant has it)
@@ -17,6 +18,7 @@ const void* tile_fn32(int v, bool warm) {
     return warm ? reinterpret_cast<const void*>(&k_tile_f32w_##id)                    \
                 : reinterpret_cast<const void*>(&k_tile_f32_##id);
     BLPG_TILE_VARIANTS(X)
+    BLPG_TILE_VARIANTS_F32(X)
 #undef X
     default: return nullptr;
   }
@@ -24,17 +26,19 @@ const void* tile_fn32(int v, bool warm) {
 
 const void* tile_fn64(int v, bool warm);  // kernel_tile64.hip
 
-constexpr int kTileVariants = 12;
-constexpr int kTileDefault = 7;  // static routing uses variants 0..6
+constexpr int kTileVariants = 14;
+constexpr int kTileDefault = 7;  // static routing by size uses variants 0..6
 
 int tile_variant_count(int) { return kTileVariants; }
 int tile_default_variants() { return kTileDefault; }
 
-TileVariant tile_variant(int, int v) {
+TileVariant tile_variant(int precision, int v) {
+  if (precision == 0 && v >= 13) return TileVariant{1, 8, 1, 1};  // FP32 only
   switch (v) {
 #define X(id, nw, tc, rpt, cpt, vr32, vr32w, vr64, vr64w, b32, b64) \
   case id: return TileVariant{nw, (nw * 64) / tc, rpt, cpt};
     BLPG_TILE_VARIANTS(X)
+    BLPG_TILE_VARIANTS_F32(X)
 #undef X
     default: return TileVariant{1, 8, 1, 1};
   }

@@ -165,11 +165,16 @@ int blpg_solve_shared_A_noalloc(int32_t m, int32_t n, const double* A, const dou
   int ncu = 0;
   if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
     return set_free_error(BLPG_E_HIP, "hipDeviceGetAttribute failed");
-  const int per_cu = tile_max_blocks_per_cu(BLPG_FP64, v);
-  if (per_cu <= 0) return set_free_error(BLPG_E_NODEVICE, "tile variant %d cannot be resident", v);
+  Route route{};
+  route.kernel = BLPG_KERNEL_TILE;
+  route.variant = v;
+  Tuner::for_many(route, m, n, BLPG_FP64, count, ncu);
+  const int per_cu = tile_max_blocks_per_cu(BLPG_FP64, route.variant);
+  if (per_cu <= 0)
+    return set_free_error(BLPG_E_NODEVICE, "tile variant %d cannot be resident", route.variant);
   TileLaunch T{};
   T.precision = BLPG_FP64;
-  T.variant = v;
+  T.variant = route.variant;
   T.desc = desc;
   T.pool = pool;
   T.spool = spool;

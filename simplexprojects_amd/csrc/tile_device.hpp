@@ -684,17 +684,28 @@ struct TileTab {
       // The block's instructions keep their order, so operands are loaded ahead of them: the
       // column, then the row in parts of at most PG entries.
       constexpr int NP = (CPT + 8) / 9, PG = (CPT + NP - 1) / NP;
-      T col[RPT];
+      // (blocks of many rows take the column in parts too, inside the row's)
+      constexpr int NK = (RPT + 7) / 8, KG = (RPT + NK - 1) / NK;
+      T col[KG];
+      auto load_col = [&](auto q) {
+        constexpr int k0 = q * KG, kn = RPT - k0 < KG ? RPT - k0 : KG;
 #pragma unroll
-      for (int k = 0; k < RPT; ++k) col[k] = cu[row_of(k)];
+        for (int k = 0; k < kn; ++k) col[k] = cu[row_of(k0 + k)];
+      };
+      if constexpr (NK == 1) load_col(std::integral_constant<int, 0>{});
       unroll<NP>([&](auto w) {
         constexpr int l0 = w * PG, ln = CPT - l0 < PG ? CPT - l0 : PG;
         T prow[ln];
+        if constexpr (NK > 1) load_col(std::integral_constant<int, 0>{});
 #pragma unroll
         for (int l = 0; l < ln; ++l) prow[l] = rb[col_of(l0 + l)];
 #pragma unroll
         for (int l = 0; l < ln; ++l) prow[l] *= rp;
-        unroll<RPT * ln>([&](auto e) { blk_fma<T, NV, el(e % RPT, l0 + e / RPT)>(col[e % RPT], prow[e / RPT]); });
+        unroll<NK>([&](auto q) {
+          constexpr int k0 = q * KG, kn = RPT - k0 < KG ? RPT - k0 : KG;
+          if constexpr (q > 0) load_col(q);
+          unroll<kn * ln>([&](auto e) { blk_fma<T, NV, el(k0 + e % kn, l0 + e / kn)>(col[e % kn], prow[e / kn]); });
+        });
       });
       publish_rhs();
       col_ready = -1;
@@ -1168,6 +1179,8 @@ __device__ __forceinline__ void tile_body(const LpDesc* __restrict__ desc, const
 // vr: vector registers left to the compiler in FP32 / FP64, cold / warm (block crash); the
 // block follows them.  Chosen so that block + vr stays within the 512 / w registers of w
 // waves per SIMD (128, 168, 256) where that admits one more LP per CU.
+// 9, 12 and 13 are the instances for many LPs (Tuner::for_many): fewer wavefronts with more of
+// the tableau each, so that one LP more fits a CU.
 //   id nw  tc rpt cpt  vr32 vr32w vr64 vr64w b32 b64
 #define BLPG_TILE_VARIANTS(X)                          \
   X(0, 1, 8, 4, 5, 76, 76, 88, 88, 1, 1)               \
@@ -1179,9 +1192,11 @@ __device__ __forceinline__ void tile_body(const LpDesc* __restrict__ desc, const
   X(6, 8, 16, 7, 13, 76, 76, 74, 74, 0, 0)             \
   X(7, 1, 8, 10, 11, 144, 144, 80, 80, 0, 0)           \
   X(8, 1, 16, 16, 7, 144, 144, 80, 80, 0, 0)           \
-  X(9, 2, 16, 14, 7, 156, 156, 80, 80, 0, 0)           \
+  X(9, 2, 16, 14, 7, 156, 156, 60, 60, 0, 0)           \
   X(10, 4, 32, 14, 4, 72, 112, 144, 144, 1, 1)         \
-  X(11, 8, 16, 4, 7, 100, 100, 72, 112, 1, 1)
+  X(11, 8, 16, 4, 7, 100, 100, 72, 112, 1, 1)          \
+  X(12, 4, 16, 11, 9, 68, 68, 58, 58, 0, 0)
+#define BLPG_TILE_VARIANTS_F32(X) X(13, 4, 16, 13, 13, 86, 86, 0, 0, 0, 0)
 
 // one kernel per variant, precision and cold / warm (the attribute takes literals only; with
 // accumulation registers in use the compiler splits its share in two, without it doubles it)

@@ -64,6 +64,7 @@ class Tuner {
   }
   void erase_check(int precision, int m, int n) { chk_.erase(key(precision, m, n)); }
   // the stored preference of a shape (false: none)
+  bool has_preference(int precision, int m, int n) const { return pref_.count(key(precision, m, n)) != 0; }
   bool get_preference(int precision, int m, int n, int& kernel, int& param, double& ms) const {
     const auto it = pref_.find(key(precision, m, n));
     if (it == pref_.end()) return false;
@@ -171,6 +172,36 @@ class Tuner {
     }
     r.kernel = BLPG_KERNEL_STREAM;
     return r;
+  }
+
+  // The instance that solves `lps` LPs of a route fastest: with more LPs than the route's own
+  // instance keeps resident without crowding, one with fewer wavefronts (and more of the
+  // tableau) each, slower per pivot but with more LPs on a CU.  Returns true and changes r
+  // where the rule applies and the shape fits.  Both sides measured on LPs of one shape, ms,
+  // before / after the line:
+  //   FP64 105x103, tile 4 / tile 9 (2-3 and 4 LPs per CU):  512 LPs 0.68 / 0.76,
+  //     768 0.89 / 0.77, 1024 1.05 / 0.80, 2048 1.87 / 1.33
+  //   FP64 174x142, tile 5 / tile 12 (1 and 2):  256 LPs 1.49 / 1.83, 512 2.61 / 2.07
+  //     (but 7.10 / 7.23 for both shapes where 512 of 205x203, which take a whole CU each,
+  //     run beside them), 768 3.65 / 3.11, 1024 4.46 / 3.67
+  //   FP32 174x142, wave 5 / tile 12 (2 and 3):  512 LPs 1.19 / 1.29, 768 1.77 / 1.38,
+  //     1024 2.05 / 1.95
+  //   FP32 205x203, wave 6 / tile 13 (1 and 2):  256 LPs 2.27 / 2.82, 512 3.58 / 2.85,
+  //     1024 6.58 / 5.05
+  static bool for_many(Route& r, int m, int n, int precision, int64_t lps, int cus) {
+    int to = -1, per_cu = 0;
+    if (precision == BLPG_FP64 && r.kernel == BLPG_KERNEL_TILE) {
+      if (r.variant == 4) { to = 9; per_cu = 2; }
+      if (r.variant == 5) { to = 12; per_cu = 2; }
+    }
+    if (precision == BLPG_FP32 && r.kernel == BLPG_KERNEL_WAVE) {
+      if (r.variant == 5) { to = 12; per_cu = 2; }
+      if (r.variant == 6) { to = 13; per_cu = 1; }
+    }
+    if (to < 0 || lps <= (int64_t)per_cu * cus || !fits_tile(to, m, n, precision)) return false;
+    r.kernel = BLPG_KERNEL_TILE;
+    r.variant = to;
+    return true;
   }
 
   static bool fits_wave(int v, int m, int n, int precision) {
