@@ -19,8 +19,8 @@ so later bins' copies overlap earlier bins' kernels) + fetch.
 The roofline object covers the dominant solve kernel (most algorithmic FLOPs): FLOPs per
 launch (sum over its LPs of pivots * 2*(m+1)*(n+1), one more row per phase-I pivot) over its
 HIP-event duration on its own stream, against the FP32 vector peak: the tableau never leaves
-registers, so the kernel is bound by the issue latency of each pivot's dependent chain
-(reductions, LDS round trips, the FMA sweep), not by HBM or MFMA.  Its HBM fraction uses
+registers (matrix-core accumulators), so the kernel is bound by the latency of each pivot's
+dependent chain (reductions, LDS round trips, the division), not by HBM or MFMA.  Its HBM fraction uses
 the per-launch traffic measured with rocprofv3 counters (profiles/traffic.json, by kernel
 route); the cycles per pivot of the bin's slowest LP bound the bin's duration.
 
@@ -48,7 +48,7 @@ PER_SHAPE = 1024
 SEED = 2
 HBM_PEAK_GBS = 8000.0
 FP32_PEAK_TFLOPS = 157.3   # MI355X published FP32 vector peak
-FP32_FMA_TFLOPS = 78.6     # one non-packed FMA per lane per clock (the kernels' only form)
+FP32_FMA_TFLOPS = 78.6     # one non-packed FMA per lane per clock
 CLOCK_GHZ = 2.4            # MI355X peak engine clock
 N_SIMD = 256 * 4           # MI355X: 256 CUs x 4 SIMDs
 KNAMES = {0: "check", 1: "stream", 2: "lds", 3: "tile", 4: "wave"}

@@ -30,7 +30,8 @@
 // division, two reductions).  FP64, one LP alone, per pivot: 0.97 us at 27x32, 1.53 at
 // 105x103, 2.13 at 174x142, 2.61 at 205x203; with every reduction on one wavefront and its
 // result broadcast (four barriers), and the block as a C++ array, 105x103 took 3.26, 174x142
-// 3.83 and 205x203 24.3 (spilled).  1024 LPs of 105x103 take 1.05 ms against 2.27.  Of 4000
+// 3.83 and 205x203 24.3 (spilled).  1024 LPs of 105x103 took 2.27 ms, now 1.05 on four
+// wavefronts each and 0.80 on two (the instance for many LPs).  Of 4000
 // cycles at 105x103 the column's way through LDS takes 880, the ratio test 970, the row 140,
 // the reciprocal and the second barrier 650, pricing 670 and the update 700.
 //
