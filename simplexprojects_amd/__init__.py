@@ -252,8 +252,8 @@ def _lp_array(lps: Sequence[LP]):
     a ctypes structure per LP, whose pointer fields cost 2 us each."""
     if not lps:
         return (_LP * 0)()
-    rows = [(lp.m, lp.n, _addr(lp.A), _addr(lp.b), _addr(lp.c), _addr(lp.sense), lp.family,
-             _addr(lp.warm_basis)) for lp in lps]
+    rows = [(lp.m, lp.n, _addr(lp.A), _addr(lp.b), _addr(lp.c), _addr(lp.sense),
+             C.c_int32(lp.family).value, _addr(lp.warm_basis)) for lp in lps]
     return (_LP * len(rows)).from_buffer(np.array(rows, dtype=_LP_DT))
 
 
