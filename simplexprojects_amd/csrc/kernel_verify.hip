@@ -103,6 +103,12 @@ struct VLayout {
 __host__ __device__ inline size_t stage_bytes(int m, int k, int tsz) {
   return (size_t)m * (size_t)(k | 1) * (size_t)(8 + tsz);
 }
+// most columns of the staged blocks: the basic structurals, and for an FP32 result one slack
+// column more, when phase I ended with every structural and x0 basic
+inline int stage_columns(int m, int n, int tsz) {
+  const int k = tsz == 4 ? n + 1 : n;
+  return m < k ? m : k;
+}
 
 // Wavefront reductions: four DPP steps leave each row of 16 lanes with its result, the four
 // rows are read back and combined; every lane ends with the same value.  (Through
@@ -231,9 +237,10 @@ __device__ int compact(int cnt, Pred pred, Key key, int* out, int* out2, int* re
 
 // Checks one LP with NT threads.  wsp: the per-LP vectors; stg: `stage_cap` bytes of LDS
 // for the staged blocks.  Returns false (and writes nothing) when the blocks do not fit
-// and `defer` is set or this is not the last tier: the caller hands the LP on.
-// LAST: the last tier, which defers nothing.  Rows of a sweep take G = NT / 128 neighbouring
-// lanes each.
+// and `defer` is set: the caller hands the LP on.  LAST: the last tier, whose sweeps also run
+// from global memory; another tier that hands nothing on (every LP of its bin fits, see
+// verify_tier_covers) fails an LP that does not fit, so that none goes without a result.
+// Rows of a sweep take G = NT / 128 neighbouring lanes each.
 template <typename TT, int NT, bool LAST>
 __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ pool,
                           const int8_t* __restrict__ spool, Out out, Check chk, double tol,
@@ -286,7 +293,7 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
       kl += (v >= 0 && v < n) ? 1 : 0;
       xl |= v == n + m ? 1 : 0;
     }
-    if (defer || !LAST) {
+    if (defer) {
       // an LP this tier hands on is decided from its basis alone (the size of its staged
       // blocks), before the rest of the bookkeeping
       const int ke = (int)bsum<NT>((double)kl, red) + ((infeas && bmax<NT>((double)xl, red) > 0) ? 1 : 0);
@@ -318,7 +325,8 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
   }
   const int kk = kq > k ? kq : k;  // columns of the staged blocks
   const bool fits = checkable && !bad && stage_bytes(m, kk, (int)sizeof(TT)) <= (size_t)stage_cap;
-  if (checkable && !bad && !fits && (defer || !LAST)) return false;
+  if (checkable && !bad && !fits && defer) return false;
+  if (!LAST && !fits) bad = 1;
   // only the last tier's kernel has the global-memory sweeps
   const bool staged = !LAST || fits;
 
@@ -993,8 +1001,8 @@ void lds_plan(int tier, int mcap, int ncap, int64_t& stage_cap, size_t& lds) {
   if (!vec_in_lds(mcap, ncap, nt)) { stage_cap = 0; lds = 0; return; }
   const size_t budget = kTierLds[tier];
   stage_cap = budget > vb ? (int64_t)(budget - vb) : 0;
-  // never more than the largest LP of the bin can use (FP64 tableau, k = min(m, n))
-  const int64_t most = (int64_t)stage_bytes(mcap, mcap < ncap ? mcap : ncap, 8);
+  // never more than the largest LP of the bin can use in either precision
+  const int64_t most = (int64_t)stage_bytes(mcap, stage_columns(mcap, ncap, 4), 8);
   if (stage_cap > most) stage_cap = most;
   lds = vb + (size_t)stage_cap;
 }
@@ -1007,10 +1015,16 @@ const void* kernel_of(int tier) {
 }
 }  // namespace
 
-bool verify_tier_used(int tier, int mcap, int ncap, int tsz) {
+// LDS bytes for the staged blocks of an LP
+int64_t verify_stage_cap(int tier, int mcap, int ncap) {
   int64_t sc;
   size_t lds;
   lds_plan(tier, mcap, ncap, sc, lds);
+  return sc;
+}
+
+bool verify_tier_used(int tier, int mcap, int ncap, int tsz) {
+  const int64_t sc = verify_stage_cap(tier, mcap, ncap);
   const int kmax = mcap < ncap ? mcap : ncap;
   if (tier == 0)  // worth a first pass when LPs with a dozen basic structurals fit
     return vec_in_lds(mcap, ncap, kTierNT[0]) && sc >= (int64_t)stage_bytes(mcap, 12, tsz);
@@ -1019,12 +1033,11 @@ bool verify_tier_used(int tier, int mcap, int ncap, int tsz) {
   return true;
 }
 
+// every LP of up to mcap x ncap fits the tier
 bool verify_tier_covers(int tier, int mcap, int ncap, int tsz) {
-  int64_t sc;
-  size_t lds;
-  lds_plan(tier, mcap, ncap, sc, lds);
   return vec_in_lds(mcap, ncap, kTierNT[tier]) &&
-         sc >= (int64_t)stage_bytes(mcap, mcap < ncap ? mcap : ncap, tsz);
+         verify_stage_cap(tier, mcap, ncap) >=
+             (int64_t)stage_bytes(mcap, stage_columns(mcap, ncap, tsz), tsz);
 }
 
 int verify_max_blocks_per_cu(int tier, int mcap, int ncap) {

@@ -103,6 +103,7 @@ struct VerifyLaunch {
 hipError_t launch_verify(const VerifyLaunch& L, hipStream_t st);
 bool verify_tier_used(int tier, int mcap, int ncap, int tsz);    // tsz: tableau element bytes
 bool verify_tier_covers(int tier, int mcap, int ncap, int tsz);  // every LP of the bin fits
+int64_t verify_stage_cap(int tier, int mcap, int ncap);  // LDS bytes for an LP's staged blocks
 int verify_max_blocks_per_cu(int tier, int mcap, int ncap);
 size_t verify_ws_stride(int mcap, int ncap);  // 0: vectors in LDS
 
