@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 import simplexprojects_amd as sa
+from tests.test_gpu_check_fit import overwrite
 
 pytestmark = pytest.mark.gpu
 
@@ -75,4 +76,29 @@ def test_options_between_solves():
         T.close()
     same(b.fetch(), ref)
     b.free()
+    S.close()
+
+
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("precision", ["fp32", "fp64"])
+@pytest.mark.parametrize("kind", ["one", "bins", "twophase", "ends", "limit", "narrow"])
+def test_later_solves_write_every_result(kind, precision, graph):
+    """The host copy holds other values before each later solve: every result of every LP is
+    the solve's own.  limit: iteration limits (FP32: all re-solved); narrow: bins of LPs with
+    fewer columns than rows, whose check has fewer tiers."""
+    if kind == "narrow":
+        batches = [[lp] * 3 for lp in lps_of("ends") if lp.n == 1]
+        batches += [sa.gen_config(2, 4, m, n, 3, batch_count=3) for m, n in [(5, 3), (60, 35), (78, 75)]]
+    else:
+        batches = [lps_of("bins" if kind == "limit" else kind)]
+    S = sa.Solver(precision=precision, verify=True, use_graph=graph, max_iter=3 if kind == "limit" else 0)
+    for lps in batches:
+        b = S.upload(lps)
+        b.solve()
+        ref = b.fetch()  # copied
+        for _ in range(2):
+            overwrite(b.fetch_raw(), lps)
+            b.solve()
+            same(b.fetch(), ref)
+        b.free()
     S.close()
