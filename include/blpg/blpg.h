@@ -166,7 +166,8 @@ int blpg_batch_repack(blpg_ctx *ctx, blpg_batch *batch, const blpg_lp *lps, int6
 
 /* Bulk results of the last blpg_batch_solve without per-LP copies: waits for the solve,
  * points `res` at host memory the batch owns (pinned), which the first fetch of a batch
- * fills with one DMA and the check of later solves as they run (without a check: the DMA).
+ * fills with one DMA and the check of later solves as they run (without a check, or fetched
+ * again: the DMA).
  * The arrays stay valid until the next solve, fetch or free of the
  * batch.  LP k's x is x[x_offset[k] .. + n_k), its basis basis[basis_offset[k] .. + m_k). */
 typedef struct {

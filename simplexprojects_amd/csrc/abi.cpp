@@ -1131,6 +1131,7 @@ int blpg_batch_fetch(blpg_ctx* ctx, blpg_batch* B, blpg_batch_results* R) {
     HIPCHK(ctx, hipMemcpyAsync(B->h_res, (char*)B->mem + B->res_off, B->res_bytes,
                                hipMemcpyDeviceToHost, ctx->stream));
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+  B->mirrored = false;  // edited below, and the caller's from here on: another fetch copies
   // the host span mirrors the device carve: int32 block, FP64 block, x pool, basis pool
   int32_t* i32 = (int32_t*)B->h_res;
   double* f64 = (double*)(B->h_res + ((char*)B->out.obj - (char*)B->out.status));

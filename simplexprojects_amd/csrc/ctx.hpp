@@ -122,7 +122,7 @@ struct blpg_batch {
   size_t res_off = 0, res_bytes = 0;  // device span of the results (one DMA)
   char* h_res = nullptr;              // pinned host copy of that span
   bool g_mirror[2] = {};              // the captured graph writes h_res itself (see Check)
-  bool mirrored = false;              // and so did the last solve
+  bool mirrored = false;              // and so did the last solve, not fetched yet
   std::vector<int64_t> x_off, basis_off;
   blpg_batch_info info{};
   hipEvent_t ev[96] = {};

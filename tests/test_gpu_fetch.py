@@ -102,3 +102,25 @@ def test_later_solves_write_every_result(kind, precision, graph):
             same(b.fetch(), ref)
         b.free()
     S.close()
+
+
+def test_a_fetch_leaves_the_solves_results_as_they_are():
+    """Options set after a solve, and what a caller writes into the fetched arrays, do not
+    reach the next fetch of the same solve, whether the check wrote them or a copy did."""
+    S = sa.Solver(precision="fp64", verify=True)
+    b = S.upload(lps_of("bins")[:40])
+    b.solve()
+    ref = b.fetch()
+    for _ in range(2):  # copied, written by the check
+        S.set(verify=0)
+        r = b.fetch()
+        assert (r.kkt_primal == -1).all() and (r.kkt_dual == -1).all()
+        S.set(verify=1)
+        same(b.fetch(), ref)
+        raw = b.fetch_raw()
+        for f in ("status", "pivots", "phase1_pivots", "fallback_used", "objective"):
+            np.ctypeslib.as_array(getattr(raw, f), shape=(40,))[:] = -77
+        same(b.fetch(), ref)
+        b.solve()
+    b.free()
+    S.close()
