@@ -771,7 +771,6 @@ static bool mirrors(const blpg_ctx* ctx, const blpg_batch* B) {
 static int enqueue_solve(blpg_ctx* ctx, blpg_batch* B, bool timing, bool copy) {
   hipStream_t st = ctx->stream;
   const int precision = ctx->opt.precision;
-  B->precision = precision;
   int32_t* q = B->d_counters;
   const int nb = (int)B->bins.size();
   double eps_d, eps_p, tol, kkt;
@@ -980,6 +979,9 @@ int blpg_batch_solve(blpg_ctx* ctx, blpg_batch* B) {
   const int g = 0;
   const bool mirror = mirrors(ctx, B);
   B->mirrored = false;
+  // what this solve's results are, for the fetches that follow it (a graph replay too)
+  B->precision = ctx->opt.precision;
+  B->checked = ctx->opt.verify || B->precision == BLPG_FP32;
   if (!ctx->opt.use_graph || B->dirty) {
     const int rc = enqueue_solve(ctx, B, true, B->dirty);
     if (!rc) B->dirty = false;
@@ -1088,7 +1090,6 @@ int blpg_batch_info_get(blpg_ctx* ctx, const blpg_batch* B, blpg_batch_info* inf
   if (!ctx || !B || !info) return BLPG_E_INVALID;
   *info = B->info;
   const int nb = (int)B->bins.size();
-  const bool checked = ctx->opt.verify || B->precision == BLPG_FP32;
   float ms = 0;
   info->verify_ms = info->fallback_ms = 0;
   info->warmstart_ms = 0;
@@ -1103,7 +1104,7 @@ int blpg_batch_info_get(blpg_ctx* ctx, const blpg_batch* B, blpg_batch_info* inf
   for (int i = 0; i < nb; ++i) {
     if (hipEventElapsedTime(&ms, B->ev[1 + 4 * i], B->ev[2 + 4 * i]) == hipSuccess)
       info->kernel_ms[i] = ms;
-    if (checked) {
+    if (B->checked) {
       if (hipEventElapsedTime(&ms, B->ev[2 + 4 * i], B->ev[3 + 4 * i]) == hipSuccess)
         info->verify_ms = std::max(info->verify_ms, (double)ms);
       if (hipEventElapsedTime(&ms, B->ev[3 + 4 * i], B->ev[4 + 4 * i]) == hipSuccess)
@@ -1114,6 +1115,12 @@ int blpg_batch_info_get(blpg_ctx* ctx, const blpg_batch* B, blpg_batch_info* inf
       hipEventElapsedTime(&ms, B->ev[kEvWsStart], B->ev[kEvWsEnd]) == hipSuccess)
     info->warmstart_ms = ms;
   return BLPG_OK;
+}
+
+// Whether a fetch reports checked results: the solve made the check (its arrays hold an
+// older solve's otherwise), and the options still ask for it (FP32: always).
+static bool reads_checked(const blpg_ctx* ctx, const blpg_batch* B) {
+  return B->checked && (ctx->opt.verify || B->precision == BLPG_FP32);
 }
 
 int blpg_batch_fetch(blpg_ctx* ctx, blpg_batch* B, blpg_batch_results* R) {
@@ -1137,7 +1144,7 @@ int blpg_batch_fetch(blpg_ctx* ctx, blpg_batch* B, blpg_batch_results* R) {
   double* f64 = (double*)(B->h_res + ((char*)B->out.obj - (char*)B->out.status));
   const double* x = (const double*)(B->h_res + ((char*)B->out.x - (char*)B->out.status));
   const int32_t* basis = (const int32_t*)(B->h_res + ((char*)B->out.basis - (char*)B->out.status));
-  const bool verified = ctx->opt.verify || B->precision == BLPG_FP32;
+  const bool verified = reads_checked(ctx, B);
   int64_t fbc = 0, piv = 0;
   for (int64_t k = 0; k < n; ++k) {
     int32_t& status = i32[k];
@@ -1197,7 +1204,7 @@ int blpg::batch_fetch_prefix(blpg_ctx* ctx, blpg_batch* B, int64_t k, blpg_batch
   HIPCHK(ctx, hipStreamSynchronize(st));
   int32_t* i32 = (int32_t*)h;
   double* f64 = (double*)(h + ((char*)B->out.obj - (char*)B->out.status));
-  const bool verified = ctx->opt.verify || B->precision == BLPG_FP32;
+  const bool verified = reads_checked(ctx, B);
   for (int64_t q = 0; q < k; ++q) {
     const int ok = i32[4 * n + q];
     if (verified && ok == 1) f64[q] = f64[2 * n + q];

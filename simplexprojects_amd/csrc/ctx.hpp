@@ -75,7 +75,8 @@ struct blpg_ctx {
 
 struct blpg_batch {
   int64_t count = 0;
-  int precision = 0;
+  int precision = 0;     // of the last solve (before one: of the upload)
+  bool checked = false;  // the last solve made the check
   std::vector<blpg::LpDesc> desc;
   int64_t pool_elems = 0, spool_elems = 0, x_elems = 0, basis_elems = 0, tab_elems = 0;
   int64_t common_elems = 0;  // pool[0, common_elems): arrays read by several bins

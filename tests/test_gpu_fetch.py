@@ -124,3 +124,53 @@ def test_a_fetch_leaves_the_solves_results_as_they_are():
         b.solve()
     b.free()
     S.close()
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_options_after_an_unchecked_solve(graph):
+    """Whether the results are checked ones, and of which precision, is a matter of the solve:
+    after an unchecked one a fetch reports no older solve's objective or residuals."""
+    lps = lps_of("bins")[:40]
+    S = sa.Solver(precision="fp64", verify=True, use_graph=graph)
+    b = S.upload(lps)
+    b.solve()
+    b.fetch()
+    S.set(verify=0, max_iter=3)
+    T = sa.Solver(precision="fp64", verify=False, max_iter=3)
+    t = T.upload(lps)
+    t.solve()
+    want = t.fetch()
+    b.solve()
+    S.set(verify=1)
+    same(b.fetch(), want)
+    assert b.info()["verify_ms"] <= 0
+    t.free()
+    b.free()
+    S.close()
+    T.close()
+
+
+def test_precisions_in_turn_around_a_repack():
+    """An FP32 graph replayed after a repacked batch was solved in FP64 without a check: FP32
+    results are checked ones whatever ran in between."""
+    lps = lps_of("bins")[:40]
+    S = sa.Solver(precision="fp32", verify=False, use_graph=True)
+    b = S.upload(lps)
+    b.solve()
+    ref = b.fetch()
+    b.solve()  # captured again, writing the host copy
+    T = sa.Solver(precision="fp64", verify=False)
+    t = T.upload(lps)
+    t.solve()
+    want = t.fetch()
+    S.set(precision="fp64")
+    b.repack(lps)
+    b.solve()
+    same(b.fetch(), want)
+    S.set(precision="fp32")
+    b.solve()
+    same(b.fetch(), ref)
+    t.free()
+    b.free()
+    S.close()
+    T.close()
