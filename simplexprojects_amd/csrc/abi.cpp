@@ -40,14 +40,14 @@ void resolve(const blpg_options& o, double& eps_d, double& eps_p, double& tol, d
 int bland_after(const blpg_options& o) { return o.bland_after > 0 ? o.bland_after : 50; }
 
 bool finite_all(const double* p, int64_t n) {
-  // x - x is +0.0 for every finite x and NaN for the others; without a branch per element
-  // the loop runs in vector registers
+  // x - x is 0 for every finite x (-0.0 where the thread rounds toward minus infinity) and
+  // NaN for the others; without a branch per element the loop runs in vector registers
   uint64_t acc = 0;
   for (int64_t i = 0; i < n; ++i) {
     const double d = p[i] - p[i];
     uint64_t u;
     std::memcpy(&u, &d, sizeof u);
-    acc |= u;
+    acc |= u << 1;
   }
   return acc == 0;
 }

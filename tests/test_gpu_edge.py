@@ -1,6 +1,7 @@
 """GPU edge cases of the drop-in path: empty and tiny batches, degenerate / cycling LPs,
 equality handling, the iteration cap, invalid input, sizes beyond the register tile, and
 the C++ drop-in program."""
+import ctypes as C
 import os
 import subprocess
 
@@ -246,3 +247,27 @@ def test_repack_packed_copy_bit_exact():
             assert np.array_equal(r.x[k], direct.x[k]), k
         batch.free()
         S.close()
+
+
+def test_upload_under_a_directed_rounding_mode():
+    """Finite inputs are finite whatever the calling thread's rounding mode (toward minus
+    infinity x - x is -0.0)."""
+    libm = C.CDLL(None)
+    lp = sa.LP(np.array([[1.0, 2.0], [3.0, 1.0]]), np.array([4.0, 5.0]), np.array([1.0, 1.0]))
+    bad = sa.LP(np.array([[1.0, np.inf], [3.0, 1.0]]), np.array([4.0, 5.0]), np.array([1.0, 1.0]))
+    S = sa.Solver(precision="fp64")
+    want = S.solve([lp])
+    mode = libm.fegetround()
+    for rounding in (0x400, 0x800, 0xC00):  # x86: down, up, toward zero
+        assert libm.fesetround(rounding) == 0
+        try:
+            b = S.upload([lp])
+            with pytest.raises(sa.BlpgError):
+                S.upload([bad])
+        finally:
+            libm.fesetround(mode)
+        b.solve()
+        r = b.fetch()
+        assert r.status[0] == want.status[0] and r.objective[0] == want.objective[0]
+        b.free()
+    S.close()
