@@ -317,10 +317,11 @@ int blpg_batch_upload(blpg_ctx* ctx, const blpg_lp* lps, int64_t count, blpg_bat
     return 3000000L + (long)r.nt * 100000L + r.bin;  // LDS: per size class
   };
   // statically routed shapes of a bin with many LPs may have a better instance (not with
-  // warm lists: those need the block crash)
+  // warm lists: those need the block crash; not in a serving arena, whose launches hold a few
+  // LPs of its many slots)
   std::vector<Route> chosen = routes;
   std::vector<uint8_t> many(count, 0);
-  if (ctx->opt.kernel == BLPG_KERNEL_AUTO && !any_warm) {
+  if (ctx->opt.kernel == BLPG_KERNEL_AUTO && !any_warm && !ctx->arena) {
     auto free_route = [&](int64_t k) {
       return !ctx->tuner.has_preference(ctx->opt.precision, B->desc[k].m, B->desc[k].n);
     };

@@ -70,6 +70,7 @@ struct blpg_ctx {
   static constexpr int kAux = 3;
   hipStream_t aux[kAux] = {};
   hipEvent_t fork = nullptr;
+  bool arena = false;  // of a serving arena: a batch's LPs are a capacity, not a load
   int64_t gen = 0;  // bumped whenever a workspace is reallocated (captured graphs go stale)
 };
 
@@ -158,6 +159,9 @@ int set_free_error(int code, const char* fmt, ...);
 
 // results of slots 0..k-1 of a batch (abi.cpp; the serving arenas use it)
 int batch_fetch_prefix(blpg_ctx* ctx, blpg_batch* B, int64_t k, blpg_batch_results* R);
+
+// info of the batch in an arena of shape (m, n) (serve.cpp; tests): which instance solves it
+int server_arena_info(blpg_server* S, int m, int n, blpg_batch_info* info);
 
 // Batches with warm-start lists crash in blocks in the register-block kernel: bins
 // routed to the accumulator kernel (which crashes one target at a time) move to the

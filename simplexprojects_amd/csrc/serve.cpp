@@ -169,6 +169,7 @@ int make_arena(blpg_server* S, Shape& sh, Arena& a) {
   o.use_graph = 1;
   int rc = blpg_create(&a.ctx, &o);
   if (rc) return rc;
+  a.ctx->arena = true;
   // Arenas of large shapes (LPs that hold a CU for milliseconds) run on three quarters of
   // the CUs, so batches of small shapes always find free CUs instead of queueing behind
   // them: a stream with a CU mask that leaves out every fourth group of 8 CUs (spread over
@@ -677,3 +678,14 @@ int blpg_server_replay(blpg_server* S, const blpg_lp* lps, const double* arrival
 }
 
 }  // extern "C"
+
+int blpg::server_arena_info(blpg_server* S, int m, int n, blpg_batch_info* info) {
+  if (!S || !info) return BLPG_E_INVALID;
+  std::lock_guard<std::mutex> lk(S->mu);
+  for (auto& kv : S->shapes)
+    if (kv.second->m == m && kv.second->n == n && !kv.second->arenas.empty()) {
+      *info = kv.second->arenas[0]->B->info;
+      return BLPG_OK;
+    }
+  return BLPG_E_INVALID;
+}

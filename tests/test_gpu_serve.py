@@ -1,6 +1,8 @@
 """GPU tests of the serving loop (blpg_server_*): single LPs of mixed shapes in, results
 equal to the batch solver's (same kernels, replayed from each shape's captured graph),
 admission against the HBM budget, and a Poisson replay with latency statistics."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -139,4 +141,27 @@ def test_server_tagged_warmstart_50k(precision):
     assert 0 < st["p50_us"] <= st["p99_us"]
     ws.close()
     Sp.close()
+    S.close()
+
+
+@pytest.mark.parametrize("precision,shape,want", [
+    ("fp64", (105, 103), (sa.KERNEL_TILE, 4)), ("fp64", (174, 142), (sa.KERNEL_TILE, 5)),
+    ("fp32", (174, 142), (sa.KERNEL_WAVE, 5)), ("fp32", (205, 203), (sa.KERNEL_WAVE, 6))])
+def test_arena_instance_goes_by_size(precision, shape, want):
+    """An arena's slots are a capacity, of which a launch usually fills a few: it takes the
+    instance of its shape, not the one for as many LPs as it has slots."""
+    info_of = getattr(sa.load_library(), "_ZN4blpg17server_arena_infoEP11blpg_serveriiP15blpg_batch_info")
+    lp = sa.gen_config(2, 7, *shape, 1, batch_count=1)[0]
+    S = sa.Solver(precision=precision)
+    srv = sa.Server(S, max_batch=1024, arenas=1, precision=precision)
+    srv.submit(lp)
+    got = []
+    while not got:
+        got = srv.poll(wait_us=100000)
+    info = sa._Info()
+    assert info_of(srv.h, C.c_int(shape[0]), C.c_int(shape[1]), C.byref(info)) == 0
+    assert (info.nbins, info.count[0]) == (1, 1024)
+    assert (info.kernel[0], info.param[0]) == want
+    assert got[0]["status"] == S.solve([lp]).status[0]
+    srv.close()
     S.close()
