@@ -51,10 +51,10 @@ def _run(cmd: list[str]) -> None:
         print(out, file=sys.stderr)
 
 
-def _check_accumulators(asm: Path) -> None:
-    """Kernels that keep tableau entries in accumulation registers name them in inline
-    assembly only; the compiler must not place values of its own there in such a kernel."""
-    kernel, own, uses = "", False, {}
+def _listing(asm: Path):
+    """(kernel, inside inline assembly?, line) of a device listing's instructions and of the
+    comments in inline assembly."""
+    kernel, own = "", False
     for line in asm.read_text().splitlines():
         if line.startswith("_Z") and ":" in line:
             kernel = line.split(":")[0]
@@ -62,22 +62,70 @@ def _check_accumulators(asm: Path) -> None:
             own = True
         elif "#ASMEND" in line:
             own = False
-        elif line.startswith("\t") and re.search(r"[ ,]a(\d|\[)", line.split(";")[0]):
-            uses.setdefault(kernel, {})[own] = line.strip()
+        elif line.startswith("\t") and (own or line[1:2] not in ".;"):
+            yield kernel, own, line.strip()
+
+
+def _registers(code: str, kind: str) -> set[int]:
+    """Numbers of the registers v.. or a.. that an instruction (or its operands) names."""
+    out = set()
+    for m in re.finditer(rf"(?<![\w.]){kind}(?:(\d+)|\[(\d+):(\d+)\])", code):
+        lo, hi = (m[1], m[1]) if m[1] else (m[2], m[3])
+        out.update(range(int(lo), int(hi) + 1))
+    return out
+
+
+def _check_accumulators(asm: Path) -> None:
+    """Kernels that keep tableau entries in accumulation registers name them in inline
+    assembly only; the compiler must not place values of its own there in such a kernel."""
+    uses: dict[str, dict[bool, str]] = {}
+    for kernel, own, line in _listing(asm):
+        if re.search(r"[ ,]a(\d|\[)", line.split(";")[0]):
+            uses.setdefault(kernel, {})[own] = line
     for k, u in uses.items():
         if len(u) == 2:
             raise RuntimeError(f"{asm.name}: in {k} the compiler uses accumulation registers "
                                f"({u[False]}): give the kernel more vector registers")
 
 
+def _check_blocks(asm: Path) -> int:
+    """Kernels that keep their block of the tableau in the registers from a number on (a
+    comment in their inline assembly names it) name them in inline assembly only: the compiler
+    must stay below it everywhere else.  Returns the number of such kernels; every kernel of
+    the listing has to be one."""
+    first: dict[str, dict[str, int]] = {}
+    used: dict[str, list[str]] = {}
+    for kernel, own, line in _listing(asm):
+        m = re.match(r"; block from v(\w+)(?: a(\w+))?", line) if own else None
+        if m:  # (decimal or hexadecimal)
+            first[kernel] = {kind: int(x, 0) for kind, x in zip("va", m.groups()) if x}
+        elif not own:
+            used.setdefault(kernel, []).append(line)
+    for kernel, lines in used.items():
+        if kernel not in first:
+            raise RuntimeError(f"{asm.name}: {kernel} does not say where its block begins")
+        for line in lines:
+            code = line.split(";")[0]
+            for kind, lim in first[kernel].items():
+                if any(r >= lim for r in _registers(code, kind)):
+                    raise RuntimeError(f"{asm.name}: in {kernel} the compiler uses registers of the "
+                                       f"block, which begins at {kind}{lim} ({line})")
+    return len(first)
+
+
+# kernels whose registers inline assembly names, and what their listing has to keep
+CHECKS = {"kernel_wave.hip": _check_accumulators, "kernel_tile.hip": _check_blocks,
+          "kernel_tile64.hip": _check_blocks}
+
+
 def _compile(src: Path) -> Path:
     obj = OBJ / (src.name + ".o")
-    if src.name == "kernel_wave.hip":
+    if src.name in CHECKS:
         _run([HIPCC, *HIPFLAGS, "--save-temps=obj", "-x", "hip", "-c", str(src), "-o", str(obj)])
         asm = list(OBJ.glob(f"{src.stem}-hip-*{ARCH}.s"))
         if len(asm) != 1:
             raise RuntimeError(f"{src.name}: no device assembly to check")
-        _check_accumulators(asm[0])
+        CHECKS[src.name](asm[0])
         return obj
     if src.suffix == ".hip" or src.name in ("abi.cpp", "simplex_shim.cpp", "warmstart.cpp",
                                             "serve.cpp", "noalloc.cpp"):

@@ -1126,9 +1126,13 @@ __device__ __forceinline__ void tile_body(const LpDesc* __restrict__ desc, const
   using Tab = TileTab<T, NW, TC, RPT, CPT, BC, NV>;
   constexpr int words = (int)sizeof(T) / 4 * RPT * CPT;
   claim<(NV + words < 256 ? NV + words : 256) - 1>();
+  // (the comment names the block's first register in the listing, for the build's check that
+  // the compiler stays below it)
   if constexpr (NV + words > 256) {
     static_assert(2 * NV + words - 256 <= 128);
-    asm volatile("" ::: "a127");
+    asm volatile("; block from v%0 a%0" ::"n"(NV) : "a127");
+  } else {
+    asm volatile("; block from v%0" ::"n"(NV));
   }
   __shared__ T colbuf[2 * Tab::RB], colupd[2 * Tab::RB], rowbuf[2 * Tab::CB], rhsbuf[Tab::RB];
   __shared__ int bs[BC ? Tab::RCAP : 1], nb[BC ? Tab::CCAP : 1], colof[BC ? Tab::RCAP + Tab::CCAP : 1];
@@ -1200,7 +1204,8 @@ __device__ __forceinline__ void tile_body(const LpDesc* __restrict__ desc, const
 #define BLPG_TILE_VARIANTS_F32(X) X(13, 4, 16, 13, 13, 86, 86, 0, 0, 0, 0)
 
 // one kernel per variant, precision and cold / warm (the attribute takes literals only; with
-// accumulation registers in use the compiler splits its share in two, without it doubles it)
+// accumulation registers in use the compiler splits its share in two, without it doubles it;
+// the build reads in the listing that it stayed below the block)
 #define BLPG_TILE_KERNEL(name, T, nw, tc, rpt, cpt, vr, words, BC)                               \
   __global__ __launch_bounds__(nw * 64)                                                          \
   __attribute__((amdgpu_num_vgpr(vr + words * rpt * cpt > 256 ? vr : vr / 2))) void name(        \
