@@ -88,6 +88,38 @@ def _check_accumulators(asm: Path) -> None:
                                f"({u[False]}): give the kernel more vector registers")
 
 
+def _check_operand_waits(asm: Path, states: int = 2) -> int:
+    """Matrix instructions and lane swaps read a vector register at the earliest `states` wait
+    states after a vector instruction wrote it.  The compiler keeps that distance between
+    instructions it knows, not where one is inline assembly, so it is read from the listing
+    (straight down: a branch only adds to it).  Returns the number of matrix instructions."""
+    count = 0
+    recent: list[tuple[int, set[int], str]] = []  # (wait states since, registers written, line)
+    for kernel, _, line in _listing(asm):
+        op, _, operands = line.split(";")[0].strip().partition(" ")
+        if not op or op.startswith("."):
+            continue
+        matrix, swap = op.startswith("v_mfma"), op.startswith("v_permlane")
+        count += matrix
+        reads = _registers(operands.partition(",")[2] if matrix else operands, "v") if matrix or swap else set()
+        for age, regs, writer in recent:
+            if regs & reads:
+                raise RuntimeError(f"{asm.name}: in {kernel} '{line}' reads a register {age} wait "
+                                   f"states after '{writer}'")
+        wait = int(operands, 0) + 1 if op == "s_nop" else 1
+        recent = [(age + wait, regs, writer) for age, regs, writer in recent if age + wait < states]
+        if op.startswith("v_") and not matrix:
+            written = operands if swap else operands.partition(",")[0]
+            recent.append((0, _registers(written, "v"), line))
+    return count
+
+
+def _check_wave(asm: Path) -> None:
+    _check_accumulators(asm)
+    if _check_operand_waits(asm) == 0:
+        raise RuntimeError(f"{asm.name}: no matrix instruction")
+
+
 def _check_blocks(asm: Path) -> int:
     """Kernels that keep their block of the tableau in the registers from a number on (a
     comment in their inline assembly names it) name them in inline assembly only: the compiler
@@ -114,7 +146,7 @@ def _check_blocks(asm: Path) -> int:
 
 
 # kernels whose registers inline assembly names, and what their listing has to keep
-CHECKS = {"kernel_wave.hip": _check_accumulators, "kernel_tile.hip": _check_blocks,
+CHECKS = {"kernel_wave.hip": _check_wave, "kernel_tile.hip": _check_blocks,
           "kernel_tile64.hip": _check_blocks}
 
 

@@ -118,7 +118,8 @@ __device__ __forceinline__ void dispatch(int k, F&& f) {
 //   acc_settle  before an access that may follow a matrix instruction (8 passes: 11 wait
 //               states until its result may be read or written)
 //   acc_ready   before matrix instructions (2 wait states after a vector write of an
-//               operand, 4 after a vector write of the execution mask)
+//               operand, 4 after a vector write of the execution mask); that no write of an
+//               operand moved behind it is read from the listing by the build
 template <int A>
 __device__ __forceinline__ float acc_get() {
   float x;

@@ -44,3 +44,36 @@ def test_kernel_that_does_not_name_its_block(tmp_path):
     f.write_text(BLOCK.format(v=80, a="", use=1, lo=2, hi=3, acc=0).replace("; block", "; no block"))
     with pytest.raises(RuntimeError, match="does not say"):
         build._check_blocks(f)
+
+
+WAITS = """
+_Z6kernelv: ; @_Z6kernelv
+\tv_cndmask_b32_e64 v17, v17, 1.0, s[8:9]
+\t;;#ASMSTART
+\t{wait}
+\t;;#ASMEND
+\t;;#ASMSTART
+\t{use}
+\t;;#ASMEND
+\ts_endpgm
+"""
+MFMA = "v_mfma_f32_16x16x1_4b_f32 a[0:15], {}, {}, a[0:15] cbsz:2 abid:0"
+
+
+@pytest.mark.parametrize("wait,use,good", [
+    ("s_nop 4", MFMA.format("v17", "v24"), True), ("s_nop 1", MFMA.format("v24", "v17"), True),
+    ("s_nop 0", MFMA.format("v17", "v24"), False), ("s_nop 0", MFMA.format("v16", "v24"), True),
+    ("v_mov_b32 v9, 0", MFMA.format("v24", "v17"), False),
+    (".set blpg_a, 3", MFMA.format("v17", "v24"), False),
+    ("s_mov_b64 exec, -1\n\ts_branch L", "v_permlane32_swap_b32_e32 v16, v17", True),
+    ("s_mov_b64 exec, -1", "v_permlane32_swap_b32_e32 v16, v17", False),
+    ("v_accvgpr_write_b32 a17, v3", "v_permlane32_swap_b32_e32 v17, v18", False),
+    ("s_nop 0", "v_add_f32_e32 v17, v17, v17", True)])
+def test_waits_before_reads_of_a_written_register(tmp_path, wait, use, good):
+    f = tmp_path / "kernel.s"
+    f.write_text(WAITS.format(wait=wait, use=use))
+    if good:
+        assert build._check_operand_waits(f) == use.startswith("v_mfma")
+    else:
+        with pytest.raises(RuntimeError, match="wait states after"):
+            build._check_operand_waits(f)
