@@ -1130,7 +1130,8 @@ __device__ __forceinline__ void tile_body(const LpDesc* __restrict__ desc, const
   // the compiler stays below it)
   if constexpr (NV + words > 256) {
     static_assert(2 * NV + words - 256 <= 128);
-    asm volatile("; block from v%0 a%0" ::"n"(NV) : "a127");
+    asm volatile("" ::: "a127");
+    asm volatile("; block from v%0 a%0" ::"n"(NV));
   } else {
     asm volatile("; block from v%0" ::"n"(NV));
   }
