@@ -337,7 +337,16 @@ int blpg_batch_upload(blpg_ctx* ctx, const blpg_lp* lps, int64_t count, blpg_bat
         many[k] = free_route(k) && Tuner::for_many(chosen[k], B->desc[k].m, B->desc[k].n, ctx->opt.precision,
                                                    fit[bin_key(routes[k])], cus);
   }
-  for (int pass = 0; pass < 2; ++pass) {
+  // a batch of too many bins goes back to the route by size, then its LDS bins (one per size
+  // class) to the HBM kernel
+  for (int pass = 0; pass < 3; ++pass) {
+    if (pass > 0) {
+      chosen = routes;
+      std::fill(many.begin(), many.end(), 0);
+    }
+    if (pass == 2)
+      for (auto& r : chosen)
+        if (r.kernel == BLPG_KERNEL_LDS) r.kernel = BLPG_KERNEL_STREAM;
     std::map<long, int> binof;
     B->bins.clear();
     for (int64_t k = 0; k < count; ++k) {
@@ -363,10 +372,6 @@ int blpg_batch_upload(blpg_ctx* ctx, const blpg_lp* lps, int64_t count, blpg_bat
       b.ccap = std::max(b.ccap, B->desc[k].n + 2);
     }
     if (B->bins.size() <= 16) break;
-    chosen = routes;
-    std::fill(many.begin(), many.end(), 0);
-    for (auto& r : chosen)
-      if (r.kernel == BLPG_KERNEL_LDS) r.kernel = BLPG_KERNEL_STREAM;
   }
   if (B->bins.size() > 16) {
     delete B;

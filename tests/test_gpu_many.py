@@ -99,3 +99,19 @@ def test_fp32_batch_solved_in_fp64(shape, count):
     b.free()
     S.close()
     T.close()
+
+
+def test_lds_bins_stay_where_the_route_by_size_has_sixteen_bins():
+    """With its other instance the batch would need a bin too many: it goes back to the route
+    by size as it stands, LDS bins included."""
+    lps = batch(174, 142, 2 * CUS + 1) + sa.gen_config(2, 7, 180, 140, 1, batch_count=1)
+    for m in (230, 250, 270, 290, 310):
+        for n in (10, 26, 42):
+            lps += sa.gen_config(2, 7, m, n, 1, batch_count=1)
+    S = sa.Solver(precision="fp64", verify=False)
+    b = S.upload(lps)
+    got = instances(b.info())
+    assert len(got) == 16 and got[-1] == (3, 5, 2 * CUS + 2)
+    assert all(kernel == 2 for kernel, _, _ in got[:-1]), got
+    b.free()
+    S.close()
