@@ -141,6 +141,12 @@ __device__ __forceinline__ double wsum(double v) {
   v += dpp_d<kDppMirror>(v);
   return (lane_d(v, 0) + lane_d(v, 16)) + (lane_d(v, 32) + lane_d(v, 48));
 }
+// |v| for the maxima that decide a result: fmax passes over a NaN, so it counts as infinite
+// (an FP32 tableau that overflowed refines to NaN throughout, and no residual is left of it)
+__device__ __forceinline__ double mag(double v) {
+  const double a = fabs(v);
+  return a <= DBL_MAX ? a : inf_of<double>();
+}
 // sum over groups of G neighbouring lanes (G = 1, 2, 4), in every lane of the group
 template <int G>
 __device__ __forceinline__ double gsum(double v) {
@@ -435,7 +441,7 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
             const double rhs = ray ? ae[p] : bp[p];
             const double val = rhs - tot - (q >= 0 ? vb[q] : 0.0);
             r[p] = val;
-            rl = fmax(rl, fabs(val));
+            rl = fmax(rl, mag(val));
           }
         }
       } else {
@@ -464,7 +470,7 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
               const double rhs = ray ? ae[p] : bp[p];
               const double val = rhs - sg(p) * tot - (q >= 0 ? vb[q] : 0.0);
               if (lane == 0) r[p] = val;
-              rl = fmax(rl, fabs(val));
+              rl = fmax(rl, mag(val));
             }
           }
         }
@@ -673,21 +679,21 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
         if (staged) {
           colsum(AB, y, k, [&](int a, double sum) {
             rho[Srow[a]] = -sum;
-            rl = fmax(rl, fabs(sum));
+            rl = fmax(rl, mag(sum));
           });
         } else {
           for (int p = tid; p < m; p += NT) w[p] = sg(p) * y[p];
           __syncthreads();
           colsum_mem(A, n, w, k, [&](int a) { return S[a]; }, [&](int a, double sum) {
             rho[Srow[a]] = -sum;
-            rl = fmax(rl, fabs(sum));
+            rl = fmax(rl, mag(sum));
           });
         }
         for (int p = tid; p < m; p += NT) {
           const int q = rowof[n + p];
           if (q >= 0) {
             rho[q] = -y[p];
-            rl = fmax(rl, fabs(y[p]));
+            rl = fmax(rl, mag(y[p]));
           }
         }
         if (tid == 0) rho[r0] = 0.0;
@@ -727,7 +733,7 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
       const double gs = am * ym;
       rp = fmax(vg / fmax(gs, DBL_MIN), yneg / fmax(ym, DBL_MIN));
       rd = -h / ((1.0 + bm) * fmax(ym, DBL_MIN));
-      ok = (ym > 0 && vg <= tol * gs && yneg <= tol * ym && -h >= sq_tol * (1.0 + bm) * ym) ? 1 : 0;
+      ok = (rres_d <= DBL_MAX && ym > 0 && ym <= DBL_MAX && vg <= tol * gs && yneg <= tol * ym && -h >= sq_tol * (1.0 + bm) * ym) ? 1 : 0;
     } else {
       // ---- x_B ----
       for (int i = tid; i < m; i += NT) x[i] = (double)T[(int64_t)(2 + i) * C];
@@ -762,7 +768,7 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
             colsum(AB, y, k, [&](int a, double sum) {
               const double val = cS[a] - sum;
               rho[Srow[a]] = val;
-              rl = fmax(rl, fabs(val));
+              rl = fmax(rl, mag(val));
             });
           } else {
             for (int p = tid; p < m; p += NT) w[p] = sg(p) * y[p];
@@ -770,14 +776,14 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
             colsum_mem(A, n, w, k, [&](int a) { return S[a]; }, [&](int a, double sum) {
               const double val = cS[a] - sum;
               rho[Srow[a]] = val;
-              rl = fmax(rl, fabs(val));
+              rl = fmax(rl, mag(val));
             });
           }
           for (int p = tid; p < m; p += NT) {
             const int q = rowof[n + p];
             if (q >= 0) {
               rho[q] = -y[p];
-              rl = fmax(rl, fabs(y[p]));
+              rl = fmax(rl, mag(y[p]));
             }
           }
           rres_d = rl;
@@ -854,7 +860,7 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
           if (tid < 128)
             for (int a = tid; a < k; a += 128) part = fma(c[S[a]], dv[Srow[a]], part);
           const double gain = (e < n ? c[e] : 0.0) - bsum<NT>(part, red);
-          good = viol <= tol * (1.0 + dmax) && rres2 <= tol * (1.0 + am * dmax) &&
+          good = dmax <= DBL_MAX && viol <= tol * (1.0 + dmax) && rres2 <= tol * (1.0 + am * dmax) &&
                  gain > tol * (1.0 + cm * (1.0 + dmax));
         }
         ok = good ? 1 : 0;

@@ -142,3 +142,36 @@ def test_singular_final_basis_falls_back_from_before_its_last_pivot():
         assert r.status[k] == cold["status"], k
         if undo:
             assert r.pivots[k] < 0.5 * cold["pivots"], (r.pivots[k], cold["pivots"])
+
+
+@pytest.mark.parametrize("config", [1, 2, 3])
+@pytest.mark.parametrize("shape", [(6, 5), (40, 34), (105, 103), (205, 203)])
+def test_tableaux_that_overflow_are_resolved(config, shape):
+    """Rows scaled by 1e39 are infinite in FP32 and the pivots turn them into NaN: a basic
+    solution that is not finite passes no check, and a reported optimum is finite.  (Not compared
+    with the unscaled LP: the tolerances are relative to max |A|.)"""
+    m, n = shape
+    lps = []
+    for k, lp in enumerate(sa.gen_config(config, 9, m, n, 8, shape_idx=1, batch_count=8)):
+        scale = np.ones(m)
+        scale[np.random.default_rng(k).permutation(m)[:1 + k * m // 8]] = 1e39
+        lps.append(sa.LP(lp.A * scale[:, None], lp.b * scale, lp.c, lp.sense))
+    S = sa.Solver(precision="fp32")
+    r = S.solve(lps)
+    S.close()
+    for k, lp in enumerate(lps):
+        o = oracle.solve(lp.A, lp.b, lp.c, lp.sense, precision="fp32", tab=True)
+        # (an infeasible or unbounded one is certified by finite duals or a finite ray alone)
+        if o["status"] == oracle.OPTIMAL and not np.isfinite(o["tab"][:, 0]).all():
+            assert r.fallback[k], k
+        if r.status[k] == sa.OPTIMAL:
+            assert np.isfinite(r.objective[k]) and np.isfinite(r.x[k]).all(), k
+
+
+def test_a_tableau_of_nan_is_no_optimum():
+    # FP32: the first row is infinite, its pivot leaves NaN everywhere; the optimum is 5 at (1, 4)
+    S = sa.Solver(precision="fp32")
+    r = S.solve([sa.LP([[1e39, 1.0], [1.0, 1.0]], [1e39, 5.0], [1.0, 1.0])])
+    S.close()
+    assert (r.status[0], r.fallback[0], r.objective[0]) == (sa.OPTIMAL, 1, 5.0)
+    assert r.x[0].tolist() == [1.0, 4.0]
