@@ -188,6 +188,12 @@ void blpg::warm_route(blpg_batch* B) {
   }
 }
 
+// whether the LDS kernel can be resident with a tableau of rcap x ccap
+static bool lds_holds(blpg_ctx* ctx, int precision, int nt, int rcap, int ccap) {
+  return stream_lds_bytes(precision, true, nt, rcap, ccap) <= ctx->tuner.lds_limit() &&
+         stream_max_blocks_per_cu(precision, true, nt, rcap, ccap) > 0;
+}
+
 static void drop_graph(blpg_batch* B, int g) {
   if (B->gexec[g]) (void)hipGraphExecDestroy(B->gexec[g]);
   if (B->graph[g]) (void)hipGraphDestroy(B->graph[g]);
@@ -351,8 +357,14 @@ int blpg_batch_upload(blpg_ctx* ctx, const blpg_lp* lps, int64_t count, blpg_bat
     B->bins.clear();
     for (int64_t k = 0; k < count; ++k) {
       const Route& r = chosen[k];
-      const long key = bin_key(r);
+      const int rcap = B->desc[k].m + 2, ccap = B->desc[k].n + 2;
+      // an LDS bin takes the LPs of its class whose largest sizes together still fit
+      long key = bin_key(r);
       auto it = binof.find(key);
+      while (r.kernel == BLPG_KERNEL_LDS && it != binof.end() &&
+             !lds_holds(ctx, ctx->opt.precision, r.nt, std::max(B->bins[it->second].rcap, rcap),
+                        std::max(B->bins[it->second].ccap, ccap)))
+        it = binof.find(key += 1000000000L);
       int bi;
       if (it == binof.end()) {
         bi = (int)B->bins.size();
@@ -368,8 +380,8 @@ int blpg_batch_upload(blpg_ctx* ctx, const blpg_lp* lps, int64_t count, blpg_bat
       }
       Bin& b = B->bins[bi];
       b.ids.push_back((int32_t)k);
-      b.rcap = std::max(b.rcap, B->desc[k].m + 2);
-      b.ccap = std::max(b.ccap, B->desc[k].n + 2);
+      b.rcap = std::max(b.rcap, rcap);
+      b.ccap = std::max(b.ccap, ccap);
     }
     if (B->bins.size() <= 16) break;
   }
@@ -602,9 +614,7 @@ static void route64(blpg_ctx* ctx, const Bin& b, Bin& f) {
   f.rcap = b.rcap; f.ccap = b.ccap; f.nt = Tuner::stream_threads(b.rcap - 2, b.ccap - 2);
   const int tv = Tuner::best_tile(b.rcap - 2, b.ccap - 2, BLPG_FP64);
   if (tv >= 0) { f.kernel = BLPG_KERNEL_TILE; f.variant = tv; }
-  else if (stream_lds_bytes(BLPG_FP64, true, f.nt, f.rcap, f.ccap) <= ctx->tuner.lds_limit() &&
-           stream_max_blocks_per_cu(BLPG_FP64, true, f.nt, f.rcap, f.ccap) > 0)
-    f.kernel = BLPG_KERNEL_LDS;
+  else if (lds_holds(ctx, BLPG_FP64, f.nt, f.rcap, f.ccap)) f.kernel = BLPG_KERNEL_LDS;
   else f.kernel = BLPG_KERNEL_STREAM;
 }
 

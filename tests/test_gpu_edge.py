@@ -271,3 +271,24 @@ def test_upload_under_a_directed_rounding_mode():
         assert r.status[0] == want.status[0] and r.objective[0] == want.objective[0]
         b.free()
     S.close()
+
+
+@pytest.mark.parametrize("kernel", ["auto", "lds"])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_shapes_that_fit_lds_one_by_one(kernel, precision):
+    """LDS bins hold a class of sizes; LPs of one class that fit a CU's LDS each, but whose
+    largest row and column counts together do not, are solved like any others."""
+    lps = [lp for m, n in [(78, 241), (66, 254), (72, 250), (78, 241)]
+           for lp in sa.gen_config(1, 3, m, n, 2, batch_count=2)]
+    S = sa.Solver(precision=precision, kernel=kernel)
+    b = S.upload(lps)
+    if precision == "fp64":
+        assert {x["kernel"] for x in b.info()["bins"]} == {sa.KERNEL_LDS}
+    b.solve()
+    r = b.fetch()
+    for k, lp in enumerate(lps):
+        o = oracle.solve(lp.A, lp.b, lp.c)
+        assert r.status[k] == o["status"]
+        assert abs(r.objective[k] - o["objective"]) <= 1e-9 * (1 + abs(o["objective"]))
+    b.free()
+    S.close()
