@@ -716,12 +716,13 @@ static int plan_solve(blpg_ctx* ctx, blpg_batch* B, SolvePlan& P) {
   for (int i = 0; i < nb; ++i) {
     const Bin& b = B->bins[i];
     const int64_t cnt = (int64_t)b.ids.size();
-    // a batch routed for FP32 and solved in FP64: instances that have no FP64 form give way
-    // to the FP64 route of their shapes
+    // a batch routed for FP32 and solved in FP64: instances that have no FP64 form, or no room
+    // for its tableau, give way to the FP64 route of their shapes
     Bin& s = P.sbins[i];
     s.kernel = b.kernel; s.variant = b.variant; s.nt = b.nt; s.rcap = b.rcap; s.ccap = b.ccap;
     if (!fp32 && ((b.kernel == BLPG_KERNEL_WAVE && wave_max_blocks_per_cu(precision, b.variant) <= 0) ||
-                  (b.kernel == BLPG_KERNEL_TILE && tile_max_blocks_per_cu(precision, b.variant) <= 0)))
+                  (b.kernel == BLPG_KERNEL_TILE && tile_max_blocks_per_cu(precision, b.variant) <= 0) ||
+                  (b.kernel == BLPG_KERNEL_LDS && !lds_holds(ctx, precision, b.nt, b.rcap, b.ccap))))
       route64(ctx, b, s);
     int rc = plan_bin(ctx, s, precision, cnt, plans[i]);
     if (rc) return rc;

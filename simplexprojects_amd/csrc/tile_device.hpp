@@ -11,6 +11,9 @@
 // amdgpu_num_vgpr attribute keeps the compiler to v[0 .. NV).  As a C++ array the block was
 // live through every branch of the state machine, and the compiler held two copies of it
 // (242 VGPRs for 98 of block, 552 bytes of scratch per lane for the 7 x 13 FP64 block).
+// What the compiler still spills of its own values, FP64: 45 registers with the 7 x 13 block,
+// 22 with 14 x 7, 62 with 11 x 9 (of the scratch accesses 1, 1 and 15 stand in the pivot loop,
+// the others in the stages around it), at most 10 elsewhere; FP32: 6 with 7 x 13.
 //
 // What the decisions need is replicated in every wavefront, in two forms: row form (lane l
 // holds rows l + 64 p: basic ids, the published column) and column form (lane l holds

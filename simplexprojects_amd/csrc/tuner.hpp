@@ -182,12 +182,19 @@ class Tuner {
   //   FP64 105x103, tile 4 / tile 9 (2-3 and 4 LPs per CU):  512 LPs 0.68 / 0.76,
   //     768 0.89 / 0.77, 1024 1.05 / 0.80, 2048 1.87 / 1.33
   //   FP64 174x142, tile 5 / tile 12 (1 and 2):  256 LPs 1.49 / 1.83, 512 2.61 / 2.07
-  //     (but 7.10 / 7.23 for both shapes where 512 of 205x203, which take a whole CU each,
-  //     run beside them), 768 3.65 / 3.11, 1024 4.46 / 3.67
+  //     (beside 512 of 205x203, which take a whole CU each, 6.9-7.1 / 6.8-7.2 for both shapes),
+  //     768 3.65 / 3.11, 1024 4.46 / 3.67
   //   FP32 174x142, wave 5 / tile 12 (2 and 3):  512 LPs 1.19 / 1.29, 768 1.77 / 1.38,
   //     1024 2.05 / 1.95
   //   FP32 205x203, wave 6 / tile 13 (1 and 2):  256 LPs 2.27 / 2.82, 512 3.58 / 2.85,
   //     1024 6.58 / 5.05
+  // Smaller shapes of the same instances (down to 70x100, 174x60, 130x90, 120x200; two data
+  // families) cross at the same counts, but for FP64 tile 5 / 12.  Alone, its shapes cross soon
+  // after one LP per CU (174x60 later): 174x142 288 LPs 1.90 / 1.85, 320 2.28 / 2.02, 448
+  // 2.43 / 2.06.  Beside LPs that take a whole CU each (205x203, 300x60) they cross between 1.5
+  // and 2 per CU: with 256 of 205x203, 288 LPs 4.06 / 4.23, 512 5.52 / 5.13.  The line is for
+  // the latter, whatever shares the batch, so 257 to 512 such LPs without them take up to 1.25
+  // times as long as they could (512 LPs of 174x142: 2.45 / 2.11).
   static bool for_many(Route& r, int m, int n, int precision, int64_t lps, int cus) {
     int to = -1, per_cu = 0;
     if (precision == BLPG_FP64 && r.kernel == BLPG_KERNEL_TILE) {

@@ -115,3 +115,22 @@ def test_lds_bins_stay_where_the_route_by_size_has_sixteen_bins():
     assert all(kernel == 2 for kernel, _, _ in got[:-1]), got
     b.free()
     S.close()
+
+
+@pytest.mark.parametrize("kernel", ["auto", "lds", "stream"])
+def test_fp32_lds_batch_solved_in_fp64(kernel):
+    """300x100 fits a CU's LDS in FP32 only."""
+    lps = sa.gen_config(2, 3, 300, 100, 3, batch_count=3)
+    S = sa.Solver(precision="fp32", kernel=kernel)
+    b = S.upload(lps)
+    assert b.info()["bins"][0]["kernel"] == (1 if kernel == "stream" else 2)
+    S.set(precision="fp64")
+    b.solve()
+    r = b.fetch()
+    T = sa.Solver(precision="fp64")
+    want = T.solve(lps)
+    for f in ("status", "pivots", "objective"):
+        assert np.array_equal(getattr(r, f), getattr(want, f)), f
+    b.free()
+    S.close()
+    T.close()
