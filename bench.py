@@ -18,11 +18,12 @@ so later bins' copies overlap earlier bins' kernels) + fetch.
 
 The roofline object covers the dominant solve kernel (most algorithmic FLOPs): FLOPs per
 launch (sum over its LPs of pivots * 2*(m+1)*(n+1), one more row per phase-I pivot) over its
-HIP-event duration on its own stream, against the FP32 vector peak: the tableau never leaves
-registers (matrix-core accumulators), so the kernel is bound by the latency of each pivot's
-dependent chain (reductions, LDS round trips, the division), not by HBM or MFMA.  Its HBM fraction uses
-the per-launch traffic measured with rocprofv3 counters (profiles/traffic.json, by kernel
-route); the cycles per pivot of the bin's slowest LP bound the bin's duration.
+HIP-event duration on its own stream, against the FP32 peak (the same for vector and matrix
+instructions).  The tableau never leaves registers (matrix-core accumulators), so the kernel
+is bound by the latency of each pivot's dependent chain (reductions, LDS round trips, the
+division), not by HBM or MFMA.  Its HBM fraction uses the per-launch traffic measured with
+rocprofv3 counters (profiles/traffic.json, by kernel route); the cycles per pivot of the bin's
+slowest LP bound the bin's duration.
 
 The CPU baseline is the oracle's FP64 replay of the same rule over all the host's cores
 (the affinity mask), on the same LPs, packed once outside the timing.
@@ -47,8 +48,8 @@ SHAPES = [(50, 48), (56, 97), (74, 83), (105, 103)]
 PER_SHAPE = 1024
 SEED = 2
 HBM_PEAK_GBS = 8000.0
-FP32_PEAK_TFLOPS = 157.3   # MI355X published FP32 vector peak
-FP32_FMA_TFLOPS = 78.6     # one non-packed FMA per lane per clock
+FP32_PEAK_TFLOPS = 157.3   # MI355X published FP32 peak, vector and matrix
+MFMA_CYCLES = 32           # of a v_mfma_f32_16x16x1_4b_f32 (2048 flops) in the matrix pipe
 CLOCK_GHZ = 2.4            # MI355X peak engine clock
 N_SIMD = 256 * 4           # MI355X: 256 CUs x 4 SIMDs
 KNAMES = {0: "check", 1: "stream", 2: "lds", 3: "tile", 4: "wave"}
@@ -414,6 +415,9 @@ def main():
     # per SIMD per 4 clocks, at the profiled clock)
     valu_frac = (prof["valu_insts"] / (N_SIMD * ms * 1e-3 * prof["clock_ghz"] * 1e9 / 4)
                  if "valu_insts" in prof else None)
+    # share of the launch in which the matrix pipes update tableaux (the same way)
+    mfma_frac = (prof["mfma_insts"] * MFMA_CYCLES / (N_SIMD * ms * 1e-3 * prof["clock_ghz"] * 1e9)
+                 if "mfma_insts" in prof else None)
     maxpiv = int(max(r32.pivots[k] for k in idx))
 
     cpu = None
@@ -445,20 +449,20 @@ def main():
                                "KKT check + FP64 fallback; inputs resident in HBM, results "
                                "to host",
                    "lps": count, "seed": SEED},
-        "roofline": {"bound": "valu", "achieved": achieved, "peak": FP32_PEAK_TFLOPS,
+        "roofline": {"bound": "latency", "achieved": achieved, "peak": FP32_PEAK_TFLOPS,
                      "unit": "TFLOP/s", "frac": achieved / FP32_PEAK_TFLOPS,
                      "traffic": traffic, "kernel": route, "launch_ms": ms,
                      "algorithmic_flops": flops[bi],
-                     "frac_of_fma_rate": achieved / FP32_FMA_TFLOPS,
                      "hbm_frac": (traffic / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS) if traffic else None,
-                     "valu_issue_frac": valu_frac,
+                     "valu_issue_frac": valu_frac, "matrix_busy_frac": mfma_frac,
                      "critical_lp_pivots": maxpiv,
                      "cycles_per_pivot_critical_lp": ms * 1e-3 * CLOCK_GHZ * 1e9 / maxpiv,
-                     "note": "latency-bound: the tableau stays in registers; frac is FLOPs "
-                             "over the FP32 vector peak (157.3 TFLOP/s); frac_of_fma_rate "
-                             "over the non-packed FMA rate (78.6 TFLOP/s); valu_issue_frac "
-                             "is the profiled VALU instruction count over the launch's "
-                             "issue slots (1024 SIMDs, one wave64 VALU op per 4 clocks)"},
+                     "note": "latency-bound: the tableau stays in registers and the longest "
+                             "LP's chain of pivots sets the time; frac is FLOPs over the FP32 "
+                             "peak (157.3 TFLOP/s); valu_issue_frac is the profiled VALU "
+                             "instruction count over the launch's issue slots (1024 SIMDs, "
+                             "one wave64 VALU op per 4 clocks), matrix_busy_frac the profiled "
+                             "matrix instructions' 32 cycles each over its cycles"},
         "cpu_baseline": cpu,
         "end_to_end": {"lps_per_s": n_good / (e2e["ms_per_step"] * 1e-3),
                        "ms_per_step": e2e["ms_per_step"], "median_ms": e2e["median_ms"],
