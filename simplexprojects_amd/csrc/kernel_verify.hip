@@ -51,6 +51,7 @@
 // (360 before), about 1.1 GB from HBM.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cfloat>
 #include <type_traits>
 
@@ -1030,8 +1031,9 @@ int64_t verify_stage_cap(int tier, int mcap, int ncap) {
 }
 
 bool verify_tier_used(int tier, int mcap, int ncap, int tsz) {
-  const int64_t sc = verify_stage_cap(tier, mcap, ncap);
+  // (what the structurals alone can use: x0's column decides nothing here)
   const int kmax = mcap < ncap ? mcap : ncap;
+  const int64_t sc = std::min(verify_stage_cap(tier, mcap, ncap), (int64_t)stage_bytes(mcap, kmax, 8));
   if (tier == 0)  // worth a first pass when LPs with a dozen basic structurals fit
     return vec_in_lds(mcap, ncap, kTierNT[0]) && sc >= (int64_t)stage_bytes(mcap, 12, tsz);
   if (tier == 1)  // worth it when a quarter of the largest blocks fit

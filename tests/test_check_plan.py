@@ -26,3 +26,12 @@ def test_a_covering_tier_holds_the_widest_blocks():
                         covered += 1
                         assert stage_bytes(m, k, tsz) <= CAP(tier, m, n), (tier, m, n, tsz)
     assert covered > 10000
+
+
+def test_x0s_column_does_not_choose_the_first_tier():
+    """The first tier is for LPs that can use a dozen staged columns: by the structurals alone."""
+    used = getattr(LIB, "_ZN4blpg16verify_tier_usedEiiii")
+    used.restype = C.c_bool
+    for tsz, dozen in ((4, 10), (8, 12)):
+        for m in (13, 20, 40):
+            assert [used(0, m, n, tsz) for n in (dozen - 1, dozen)] == [False, True], (m, tsz)
