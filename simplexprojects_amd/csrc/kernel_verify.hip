@@ -142,12 +142,10 @@ __device__ __forceinline__ double wsum(double v) {
   v += dpp_d<kDppMirror>(v);
   return (lane_d(v, 0) + lane_d(v, 16)) + (lane_d(v, 32) + lane_d(v, 48));
 }
-// |v| for the maxima that decide a result: fmax passes over a NaN, so it counts as infinite
-// (an FP32 tableau that overflowed refines to NaN throughout, and no residual is left of it)
-__device__ __forceinline__ double mag(double v) {
-  const double a = fabs(v);
-  return a <= DBL_MAX ? a : inf_of<double>();
-}
+// fmax passes over a NaN, and an FP32 tableau that overflowed refines to NaN throughout: the last
+// residuals of a refinement are looked at once more, each on its own.  (Counted as infinite in
+// the sweeps themselves, they cost 1-2% of the check.)
+__device__ __forceinline__ bool finite(double v) { return fabs(v) <= DBL_MAX; }
 // sum over groups of G neighbouring lanes (G = 1, 2, 4), in every lane of the group
 template <int G>
 __device__ __forceinline__ double gsum(double v) {
@@ -442,7 +440,7 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
             const double rhs = ray ? ae[p] : bp[p];
             const double val = rhs - tot - (q >= 0 ? vb[q] : 0.0);
             r[p] = val;
-            rl = fmax(rl, mag(val));
+            rl = fmax(rl, fabs(val));
           }
         }
       } else {
@@ -471,7 +469,7 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
               const double rhs = ray ? ae[p] : bp[p];
               const double val = rhs - sg(p) * tot - (q >= 0 ? vb[q] : 0.0);
               if (lane == 0) r[p] = val;
-              rl = fmax(rl, mag(val));
+              rl = fmax(rl, fabs(val));
             }
           }
         }
@@ -680,21 +678,21 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
         if (staged) {
           colsum(AB, y, k, [&](int a, double sum) {
             rho[Srow[a]] = -sum;
-            rl = fmax(rl, mag(sum));
+            rl = fmax(rl, fabs(sum));
           });
         } else {
           for (int p = tid; p < m; p += NT) w[p] = sg(p) * y[p];
           __syncthreads();
           colsum_mem(A, n, w, k, [&](int a) { return S[a]; }, [&](int a, double sum) {
             rho[Srow[a]] = -sum;
-            rl = fmax(rl, mag(sum));
+            rl = fmax(rl, fabs(sum));
           });
         }
         for (int p = tid; p < m; p += NT) {
           const int q = rowof[n + p];
           if (q >= 0) {
             rho[q] = -y[p];
-            rl = fmax(rl, mag(y[p]));
+            rl = fmax(rl, fabs(y[p]));
           }
         }
         if (tid == 0) rho[r0] = 0.0;
@@ -721,6 +719,7 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
       for (int p = tid; p < m; p += NT) {
         const double yp = y[p];
         if (!is_eq(p)) yneg = fmax(yneg, -yp);
+        if (!finite(rho[p])) yneg = inf_of<double>();
         w[p] = sg(p) * (is_eq(p) ? yp : fmax(yp, 0.0));
       }
       __syncthreads();
@@ -734,7 +733,7 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
       const double gs = am * ym;
       rp = fmax(vg / fmax(gs, DBL_MIN), yneg / fmax(ym, DBL_MIN));
       rd = -h / ((1.0 + bm) * fmax(ym, DBL_MIN));
-      ok = (rres_d <= DBL_MAX && ym > 0 && ym <= DBL_MAX && vg <= tol * gs && yneg <= tol * ym && -h >= sq_tol * (1.0 + bm) * ym) ? 1 : 0;
+      ok = (ym > 0 && finite(ym) && vg <= tol * gs && yneg <= tol * ym && -h >= sq_tol * (1.0 + bm) * ym) ? 1 : 0;
     } else {
       // ---- x_B ----
       for (int i = tid; i < m; i += NT) x[i] = (double)T[(int64_t)(2 + i) * C];
@@ -747,8 +746,10 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
         const double xv = x[i];
         if (v < n) pv = fmax(pv, -xv);
         else pv = fmax(pv, is_eq(v - n) ? fabs(xv) : -xv);
+        if (!finite(r[i])) pv = inf_of<double>();
       }
       pv = bmax<NT>(pv, red);
+      if (!finite(pv)) rres = pv;
       rp = fmax(pv, rres) / (1.0 + bm + am * xm);
       const bool pconv = rres <= sq_tol * (1.0 + bm);
       keep_basis = keep_basis || pconv;
@@ -769,7 +770,7 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
             colsum(AB, y, k, [&](int a, double sum) {
               const double val = cS[a] - sum;
               rho[Srow[a]] = val;
-              rl = fmax(rl, mag(val));
+              rl = fmax(rl, fabs(val));
             });
           } else {
             for (int p = tid; p < m; p += NT) w[p] = sg(p) * y[p];
@@ -777,14 +778,14 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
             colsum_mem(A, n, w, k, [&](int a) { return S[a]; }, [&](int a, double sum) {
               const double val = cS[a] - sum;
               rho[Srow[a]] = val;
-              rl = fmax(rl, mag(val));
+              rl = fmax(rl, fabs(val));
             });
           }
           for (int p = tid; p < m; p += NT) {
             const int q = rowof[n + p];
             if (q >= 0) {
               rho[q] = -y[p];
-              rl = fmax(rl, mag(y[p]));
+              rl = fmax(rl, fabs(y[p]));
             }
           }
           rres_d = rl;
@@ -813,8 +814,10 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
         a_columns([&](int j, double tot) {
           if (rowof[j] < 0) dvv = fmax(dvv, c[j] - tot);
         });
-        for (int p = tid; p < m; p += NT)
+        for (int p = tid; p < m; p += NT) {
           if (colp[p] >= 0 && !is_eq(p)) dvv = fmax(dvv, -y[p]);
+          if (!finite(rho[p])) dvv = inf_of<double>();
+        }
         rd = fmax(bmax<NT>(dvv, red), rres_d) / (1.0 + cm + am * ym);
         dconv = rres_d <= sq_tol * (1.0 + cm);
       }
@@ -855,13 +858,14 @@ __device__ bool verify_lp(int lp, const LpDesc& D, const double* __restrict__ po
           for (int i = tid; i < m; i += NT) {
             const int bv = bs[i];
             viol = fmax(viol, (bv >= n && is_eq(bv - n)) ? fabs(dv[i]) : dv[i]);
+            if (!finite(r[i])) viol = inf_of<double>();
           }
           viol = bmax<NT>(viol, red);
           double part = 0;
           if (tid < 128)
             for (int a = tid; a < k; a += 128) part = fma(c[S[a]], dv[Srow[a]], part);
           const double gain = (e < n ? c[e] : 0.0) - bsum<NT>(part, red);
-          good = dmax <= DBL_MAX && viol <= tol * (1.0 + dmax) && rres2 <= tol * (1.0 + am * dmax) &&
+          good = finite(dmax) && viol <= tol * (1.0 + dmax) && rres2 <= tol * (1.0 + am * dmax) &&
                  gain > tol * (1.0 + cm * (1.0 + dmax));
         }
         ok = good ? 1 : 0;
